@@ -123,6 +123,22 @@ struct SpModel {
     double t_coeff[kSpMaxTerms];
     int pc[kSpMaxSpecies][kSpMaxPatches];  // patch multiplicities per species
     double B2[kSpMaxSpecies][kSpMaxSpecies];
+    double delta[kSpMaxPatches][kSpMaxPatches];  // bonding volumes between patch types some species carries
+};
+// species and patch types up to which a generic model runs with its vectors in
+// registers (statically indexed) and the accelerated mass-action solve
+constexpr int kSpSmall = 4;
+// the model's numbers of a system with at most kSpSmall species and patch types
+// (Saleh, Ricci, small generic models): a kernel argument, so a kernel's scalar
+// loads of it are few and consecutive
+struct SpSmallModel {
+    int model, S, P;
+    double k[kSpSmall];
+    int val[3], lh;
+    double sB2, sB3, dAA, dBB, rB2, d00, d12;
+    int pc[kSpSmall][kSpSmall];
+    double B2[kSpSmall][kSpSmall];
+    double dl[kSpSmall][kSpSmall];             // bonding volumes between patch types
 };
 void sp_build_model(const ch_species_model &in, SpModel &m);
 struct SpArgs {
@@ -137,6 +153,7 @@ struct SpArgs {
     void *spec[2];          // hat (T2) scratch
     int64_t bins, hat;
 };
+// X = 1 everywhere, then one model evaluation (Generic; nothing for the others)
 hipError_t sp_warm(const SpArgs &a, hipStream_t s);
 hipError_t sp_step_stencil(const SpArgs &a, int integrator, hipStream_t s);
 hipError_t sp_step_spectral(const SpArgs &a, const SpectralArgs &sa, hipStream_t s);

@@ -13,6 +13,7 @@
 // log_series (ch_device.h, within 2 ulp); the free energy keeps the library's.
 //
 // Integrators over species-major fields rho[s * bins + i]:
+//   (generic models of at most 4 species and 4 patch types: small_update_X)
 //   euler / euler_mobility: k_sp_mu (mobility from the previous X, X update,
 //     f', mu_s = f'_s - 2 k_s lap rho_s) then k_sp_update (rho_s += dt M lap mu_s,
 //     or the flux form with M_s per species), in place: 2 launches per step
@@ -33,6 +34,7 @@ using C2 = typename Complex<T>::type;
 
 constexpr int kSpBlocks = 2048;
 
+// more than kSpSmall species or patch types, and the free energy: the bare sweeps
 __device__ void generic_update_X(const SpModel &m, const double *rhos, double *X) {
 #pragma clang fp contract(off)
     for(int iter = 0; iter < 10000; iter++) {
@@ -53,7 +55,8 @@ __device__ void generic_update_X(const SpModel &m, const double *rhos, double *X
     }
 }
 
-__device__ double saleh_contribution(const SpModel &m, const double *rhos, int species) {
+// ln X of one Saleh bonding site; rf = delta (valence rho + lh rho_linker)
+__device__ __forceinline__ double saleh_log_X(const SpSmallModel &m, const double (&rhos)[3], int species) {
 #pragma clang fp contract(off)
     const double delta = species == 0 ? m.dAA : m.dBB;
     const double rho_factor = delta * (m.val[species] * rhos[species] + m.lh * rhos[2]);
@@ -61,50 +64,168 @@ __device__ double saleh_contribution(const SpModel &m, const double *rhos, int s
     return rho_factor >= 0 ? log_series(X) : 0.0;
 }
 
-// f' of every species at one cell; X (Generic) in/out
-__device__ void sp_fprime(const SpModel &m, const double *rhos, double *X, double *out) {
+// 1 / d for d in [1, 2^100): the hardware reciprocal and two Newton steps, within
+// 1 ulp in five dependent operations where the IEEE division takes about ten
+__device__ __forceinline__ double recip(double d) {
+    double r = __builtin_amdgcn_rcp(d);
+    r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+    return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+}
+
+// generic_update_X's sweeps, on X_p = 1 / (1 + sum_q a_pq X_q)
+template <int P, bool SHORT>
+__device__ __forceinline__ void small_sweeps(const double (&a)[P][P], double (&X)[P]) {
 #pragma clang fp contract(off)
-    const int S = m.S;
-    double logX[kSpMaxPatches];
-    if(m.model == CH_GENERIC_WERTHEIM) {
-        generic_update_X(m, rhos, X);
-        for(int i = 0; i < m.P; i++) logX[i] = log_series(X[i]);
+#pragma unroll 1
+    for(int iter = 0; iter < 10000; iter++) {
+        double max_delta = 0.0;
+#pragma unroll
+        for(int p = 0; p < P; p++) {
+            double sum = 1.0;
+#pragma unroll
+            for(int q = 0; q < P; q++) sum = __builtin_fma(a[p][q], X[q], sum);
+            const double new_X = SHORT ? recip(sum) : 1.0 / sum;
+            const double d = fabs(new_X - X[p]);
+            max_delta = (max_delta < d) ? d : max_delta;
+            X[p] = new_X;
+        }
+        if(max_delta < 1e-8) return;
     }
-    for(int s = 0; s < S; s++) {
-        out[s] = 0.0;
-        if(rhos[s] == 0.) continue;
-        double rho_tot = 0.;
-        for(int t = 0; t < S; t++) rho_tot += rhos[t];
-        double ref, bond = 0.0;
-        if(m.model == CH_SALEH_WERTHEIM) {
-            ref = log_series(rhos[s]) + 2.0 * m.sB2 * rho_tot + 3.0 * m.sB3 * (rho_tot * rho_tot);
-            if(s == 0) bond = m.val[0] * saleh_contribution(m, rhos, 0);
-            else if(s == 1) bond = m.val[1] * saleh_contribution(m, rhos, 1);
-            else bond = m.lh * (saleh_contribution(m, rhos, 0) + saleh_contribution(m, rhos, 1));
+}
+
+// generic_update_X for a small model: the same sweeps in the same order with
+// a_pq = delta_pq sum_s rho_s n_sq formed once per cell.  A cell needs some 200
+// sweeps from X = 1 and a few per time step, each a dependent chain, so the
+// chain's length and its branches are what count: P^2 fused terms, the short
+// reciprocal and no branch per sweep, where the general form tests and indexes
+// every (species, patch) pair (2D N = 256, 3 species, 2 patch types, FP64: see
+// k_sp_mu).  Densities that are negative, NaN or huge take the IEEE division.
+// Newton steps between the sweeps reach the fixed point in 3 sweeps, but not
+// the state at which the reference's rule stops: up to 8e-8 away for slowly
+// contracting topologies.
+template <int P>
+__device__ __forceinline__ void small_update_X(const SpSmallModel &m, const double (&rhos)[kSpSmall], double (&X)[P]) {
+#pragma clang fp contract(off)
+    double a[P][P];
+    bool tame = true;
+#pragma unroll
+    for(int q = 0; q < P; q++) {
+        double n = 0.0;
+#pragma unroll
+        for(int s = 0; s < kSpSmall; s++)
+            if(s < m.S) n += rhos[s] * (double)m.pc[s][q];
+#pragma unroll
+        for(int p = 0; p < P; p++) {
+            a[p][q] = m.dl[p][q] * n;
+            tame = tame && a[p][q] >= 0.0 && a[p][q] < 0x1p90;
         }
-        else if(m.model == CH_RICCI_WERTHEIM) {
-            ref = log_series(rhos[s]) + 2.0 * m.rB2 * rho_tot;
-            const double A = rhos[1] * m.d12, B = rhos[0] * m.d12;
-            if(s == 0) {
-                const double X0 = (-1 + sqrt((1 + 12 * rhos[0] * m.d00))) / (6 * rhos[0] * m.d00);
-                const double u = 1 + 2 * A - B;
-                const double X1 = (B - 1 - 2 * A + sqrt(u * u + 4 * B)) / (2 * B);
-                bond = 3 * log_series(X0) + log_series(X1);
-            }
-            else {
-                const double v = B - 2 * A + 1;
-                const double X2 = (-B + 2 * A - 1 + sqrt(v * v + 8 * A)) / (4 * A);
-                bond = 2 * log_series(X2);
-            }
+    }
+    if(tame) small_sweeps<P, true>(a, X);
+    else small_sweeps<P, false>(a, X);
+}
+
+// A model whose species and patch vectors have sizes known at compile time
+// keeps them in registers; the others (dyn: more than kSpSmall species or patch
+// types, or a patch type that no species carries) index them at run time.  S, P: sizes of the vectors; exact: S is the
+// number of species (else it is m.S <= S).
+struct SalehModel {
+    using M = SpSmallModel;
+    static constexpr int model = CH_SALEH_WERTHEIM, S = 3, P = 1;
+    static constexpr bool exact = true, dyn = false;
+};
+struct RicciModel {
+    using M = SpSmallModel;
+    static constexpr int model = CH_RICCI_WERTHEIM, S = 2, P = 1;
+    static constexpr bool exact = true, dyn = false;
+};
+template <int P_>
+struct SmallModel {
+    using M = SpSmallModel;
+    static constexpr int model = CH_GENERIC_WERTHEIM, S = kSpSmall, P = P_;
+    static constexpr bool exact = false, dyn = false;
+};
+struct LargeModel {
+    using M = const SpModel *;
+    static constexpr int model = CH_GENERIC_WERTHEIM, S = kSpMaxSpecies, P = kSpMaxPatches;
+    static constexpr bool dyn = true;
+};
+__device__ __forceinline__ const SpSmallModel &model_of(const SpSmallModel &m) { return m; }
+__device__ __forceinline__ const SpModel &model_of(const SpModel *const &m) { return *m; }
+
+// f(s) for every species s of the model (unrolled where the sizes are static)
+template <class MD, class M, typename F>
+__device__ __forceinline__ void each_species(const M &m, F &&f) {
+    if constexpr(MD::dyn) {
+        for(int s = 0; s < m.S; s++) f(s);
+    }
+    else {
+#pragma unroll
+        for(int s = 0; s < MD::S; s++)
+            if(MD::exact || s < m.S) f(s);
+    }
+}
+// f(q) for every patch type of a generic model
+template <class MD, class M, typename F>
+__device__ __forceinline__ void each_patch(const M &m, F &&f) {
+    if constexpr(MD::model != CH_GENERIC_WERTHEIM) return;
+    else if constexpr(MD::dyn) {
+        for(int q = 0; q < m.P; q++) f(q);
+    }
+    else {
+#pragma unroll
+        for(int q = 0; q < MD::P; q++) f(q);
+    }
+}
+
+template <class MD, class M>
+__device__ __forceinline__ void update_X(const M &m, const double (&rhos)[MD::S], double (&X)[MD::P]) {
+    if constexpr(MD::dyn) generic_update_X(m, rhos, X);
+    else if constexpr(MD::model == CH_GENERIC_WERTHEIM) small_update_X<MD::P>(m, rhos, X);
+}
+
+// f' of every species at one cell; X (Generic) in/out
+template <class MD, class M>
+__device__ __forceinline__ void sp_fprime(const M &m, const double (&rhos)[MD::S], double (&X)[MD::P],
+                                          double (&out)[MD::S]) {
+#pragma clang fp contract(off)
+    double rho_tot = 0.;
+    each_species<MD>(m, [&](int s) { rho_tot += rhos[s]; });
+    if constexpr(MD::model == CH_SALEH_WERTHEIM) {
+        const double c0 = saleh_log_X(m, rhos, 0), c1 = saleh_log_X(m, rhos, 1);
+        const double bond[3] = {m.val[0] * c0, m.val[1] * c1, m.lh * (c0 + c1)};
+#pragma unroll
+        for(int s = 0; s < 3; s++) {
+            const double ref = log_series(rhos[s]) + 2.0 * m.sB2 * rho_tot + 3.0 * m.sB3 * (rho_tot * rho_tot);
+            out[s] = rhos[s] == 0. ? 0.0 : ref + bond[s];
         }
-        else {
-            double B2c = 0.;
-            for(int o = 0; o < S; o++) B2c += 2.0 * rhos[o] * m.B2[s][o];
-            ref = log_series(rhos[s]) + B2c;
-            for(int q = 0; q < m.P; q++)
+    }
+    else if constexpr(MD::model == CH_RICCI_WERTHEIM) {
+        const double A = rhos[1] * m.d12, B = rhos[0] * m.d12;
+        const double X0 = (-1 + sqrt((1 + 12 * rhos[0] * m.d00))) / (6 * rhos[0] * m.d00);
+        const double u = 1 + 2 * A - B;
+        const double X1 = (B - 1 - 2 * A + sqrt(u * u + 4 * B)) / (2 * B);
+        const double v = B - 2 * A + 1;
+        const double X2 = (-B + 2 * A - 1 + sqrt(v * v + 8 * A)) / (4 * A);
+        const double bond[2] = {3 * log_series(X0) + log_series(X1), 2 * log_series(X2)};
+#pragma unroll
+        for(int s = 0; s < 2; s++) {
+            const double ref = log_series(rhos[s]) + 2.0 * m.rB2 * rho_tot;
+            out[s] = rhos[s] == 0. ? 0.0 : ref + bond[s];
+        }
+    }
+    else {
+        update_X<MD>(m, rhos, X);
+        double logX[MD::P];
+        each_patch<MD>(m, [&](int q) { logX[q] = log_series(X[q]); });
+        each_species<MD>(m, [&](int s) {
+            double B2c = 0., bond = 0.;
+            each_species<MD>(m, [&](int o) { B2c += 2.0 * rhos[o] * m.B2[s][o]; });
+            const double ref = log_series(rhos[s]) + B2c;
+            each_patch<MD>(m, [&](int q) {
                 if(m.pc[s][q] > 0) bond += m.pc[s][q] * logX[q];
-        }
-        out[s] = ref + bond;
+            });
+            out[s] = rhos[s] == 0. ? 0.0 : ref + bond;
+        });
     }
 }
 
@@ -158,8 +279,24 @@ __device__ double sp_bulk(const SpModel &m, double dcf, const double *rhos) {
     return f_ref + bond;
 }
 
+// x^n, n >= 1 (patch multiplicities are small): products up to 4, binary powers above
+__device__ __forceinline__ double int_power(double x, int n) {
+#pragma clang fp contract(off)
+    const double x2 = x * x;
+    if(n <= 4) return n == 1 ? x : (n == 2 ? x2 : (n == 3 ? x2 * x : x2 * x2));
+    double r = 1.0;
+    for(;;) {
+        if(n & 1) r *= x;
+        n >>= 1;
+        if(n == 0) return r;
+        x *= x;
+    }
+}
+
 // mobility of species s (RegularisedMobility.h:26-33; GenericWertheim.cpp:276-291)
-__device__ double sp_mobility(const Params &p, const SpModel &m, int mob, int s, double r, const double *X) {
+template <class MD, class M>
+__device__ __forceinline__ double sp_mobility(const Params &p, const M &m, int mob, int s, double r,
+                                              const double (&X)[MD::P]) {
 #pragma clang fp contract(off)
     switch(mob) {
     case CH_MOB_CONSTANT: return p.M;
@@ -167,8 +304,9 @@ __device__ double sp_mobility(const Params &p, const SpModel &m, int mob, int s,
     case CH_MOB_LINEAR: return p.M * r / p.rho_ref;
     default: {
         double D = p.M;
-        for(int q = 0; q < m.P; q++)
-            if(m.pc[s][q] > 0) D *= pow(X[q], (double)m.pc[s][q]);
+        each_patch<MD>(m, [&](int q) {
+            if(m.pc[s][q] > 0) D *= int_power(X[q], m.pc[s][q]);
+        });
         return r * D;
     }
     }
@@ -197,95 +335,111 @@ __device__ __forceinline__ void neighbours(const Params &p, int64_t i, int64_t (
 
 #define SP_CELLS for(int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < bins; i += (int64_t)gridDim.x * 256)
 
-// X update only: the model evaluation of CahnHilliard.cpp:226-228 at set-up
-template <typename T>
+// the densities and X of cell i
+template <class MD, class M, typename T>
+__device__ __forceinline__ void load_cell(const M &m, const T *__restrict__ rho, const double *__restrict__ Xf,
+                                          int64_t i, int64_t bins, double (&rhos)[MD::S], double (&X)[MD::P]) {
+    each_species<MD>(m, [&](int s) { rhos[s] = (double)rho[s * bins + i]; });
+    each_patch<MD>(m, [&](int q) { X[q] = Xf[q * bins + i]; });
+}
+
+// X = 1 (GenericWertheim.cpp:252-254), then the model evaluation of
+// CahnHilliard.cpp:226-228 at set-up
+template <typename T, class MD>
 __global__ __launch_bounds__(256) void k_sp_warm(const T *__restrict__ rho, double *__restrict__ Xf,
-                                                 const SpModel *__restrict__ mp, int64_t bins) {
-    const SpModel &m = *mp;
+                                                 typename MD::M arg, int64_t bins) {
+    const auto &m = model_of(arg);
     SP_CELLS {
-        double rhos[kSpMaxSpecies], X[kSpMaxPatches], out[kSpMaxSpecies];
-        for(int s = 0; s < m.S; s++) rhos[s] = (double)rho[s * bins + i];
-        for(int q = 0; q < m.P; q++) X[q] = Xf[q * bins + i];
-        sp_fprime(m, rhos, X, out);
-        for(int q = 0; q < m.P; q++) Xf[q * bins + i] = X[q];
+        double rhos[MD::S], X[MD::P];
+        each_species<MD>(m, [&](int s) { rhos[s] = (double)rho[s * bins + i]; });
+        each_patch<MD>(m, [&](int q) { X[q] = 1.0; });
+        update_X<MD>(m, rhos, X);
+        each_patch<MD>(m, [&](int q) { Xf[q * bins + i] = X[q]; });
     }
 }
 
-// mu_s = f'_s - 2 k_s lap rho_s (and M_s from the X before this evaluation)
-template <typename T, int DIMS>
+// mu_s = f'_s - 2 k_s lap rho_s (and M_s from the X before this evaluation).
+// One cell per thread: at the sizes in use (2D N = 256: one wave per SIMD) the
+// model's dependent divisions, roots and logarithms bound it, so the loads are
+// all issued first, the species are unrolled to overlap their chains and nothing
+// branches on the model's sizes (SmallModel): 7.7 us at 2D N = 256 FP64 with 3
+// species, 2 patch types and the free-energy mobility, 16.1 with run-time
+// indexed vectors and pow() (k_sp_warm: 41 us, 276).
+template <typename T, int DIMS, class MD>
 __global__ __launch_bounds__(256) void k_sp_mu(const T *__restrict__ rho, double *__restrict__ Xf, T *__restrict__ mu,
-                                               T *__restrict__ mobf, Params p, const SpModel *__restrict__ mp,
+                                               T *__restrict__ mobf, Params p, typename MD::M arg,
                                                int64_t bins, int mob) {
 #pragma clang fp contract(off)
-    const SpModel &m = *mp;
+    const auto &m = model_of(arg);
     SP_CELLS {
-        double rhos[kSpMaxSpecies], X[kSpMaxPatches], f[kSpMaxSpecies];
-        for(int s = 0; s < m.S; s++) rhos[s] = (double)rho[s * bins + i];
-        for(int q = 0; q < m.P; q++) X[q] = Xf[q * bins + i];
-        if(mob >= 0)
-            for(int s = 0; s < m.S; s++) mobf[s * bins + i] = (T)sp_mobility(p, m, mob, s, rhos[s], X);
-        sp_fprime(m, rhos, X, f);
-        for(int q = 0; q < m.P; q++) Xf[q * bins + i] = X[q];
+        double rhos[MD::S], X[MD::P], f[MD::S];
+        load_cell<MD>(m, rho, Xf, i, bins, rhos, X);
         int64_t nm[DIMS], nq[DIMS];
         neighbours<DIMS>(p, i, nm, nq);
         const T inv_dx2 = (T)p.inv_dx2;
-        for(int s = 0; s < m.S; s++) {
+        T lap[MD::S];
+        each_species<MD>(m, [&](int s) {
             const T *r = rho + s * bins;
             T a[DIMS], b[DIMS];
+#pragma unroll
             for(int d = 0; d < DIMS; d++) {
                 a[d] = r[nm[d]];
                 b[d] = r[nq[d]];
             }
-            const T lap = laplacian<T, DIMS>(r[i], a, b, inv_dx2);
-            mu[s * bins + i] = (T)f[s] - (T)(2 * m.k[s]) * lap;
-        }
+            lap[s] = laplacian<T, DIMS>((T)rhos[s], a, b, inv_dx2);
+        });
+        if(mob >= 0)
+            each_species<MD>(m, [&](int s) { mobf[s * bins + i] = (T)sp_mobility<MD>(p, m, mob, s, rhos[s], X); });
+        sp_fprime<MD>(m, rhos, X, f);
+        each_patch<MD>(m, [&](int q) { Xf[q * bins + i] = X[q]; });
+        each_species<MD>(m, [&](int s) { mu[s * bins + i] = (T)f[s] - (T)(2 * m.k[s]) * lap[s]; });
     }
 }
 
-// rho_s += dt M lap mu_s (euler) or dt div J_s (euler_mobility), in place
+// rho_s += dt M lap mu_s (euler) or dt div J_s (euler_mobility), in place; one
+// species per grid row, so a cell's species run in different blocks
 template <typename T, int DIMS, bool EM>
 __global__ __launch_bounds__(256) void k_sp_update(T *__restrict__ rho, const T *__restrict__ mu,
-                                                   const T *__restrict__ mobf, Params p, int S, int64_t bins) {
+                                                   const T *__restrict__ mobf, Params p, int64_t bins) {
 #pragma clang fp contract(off)
+    const int64_t base = (int64_t)blockIdx.y * bins;
+    const T *u = mu + base, *M = mobf + base;
+    T *r = rho + base;
     SP_CELLS {
         int64_t nm[DIMS], nq[DIMS];
         neighbours<DIMS>(p, i, nm, nq);
-        for(int s = 0; s < S; s++) {
-            const T *u = mu + s * bins;
-            T a[DIMS], b[DIMS];
+        T a[DIMS], b[DIMS];
+#pragma unroll
+        for(int d = 0; d < DIMS; d++) {
+            a[d] = u[nm[d]];
+            b[d] = u[nq[d]];
+        }
+        if constexpr(!EM) {
+            r[i] = euler_update<T, DIMS>(p, r[i], u[i], a, b);
+        }
+        else {
+            T Ma[DIMS], Mb[DIMS];
+#pragma unroll
             for(int d = 0; d < DIMS; d++) {
-                a[d] = u[nm[d]];
-                b[d] = u[nq[d]];
+                Ma[d] = M[nm[d]];
+                Mb[d] = M[nq[d]];
             }
-            T *r = rho + s * bins;
-            if constexpr(!EM) {
-                r[i] = euler_update<T, DIMS>(p, r[i], u[i], a, b);
-            }
-            else {
-                const T *M = mobf + s * bins;
-                T Ma[DIMS], Mb[DIMS];
-                for(int d = 0; d < DIMS; d++) {
-                    Ma[d] = M[nm[d]];
-                    Mb[d] = M[nq[d]];
-                }
-                r[i] = mobility_update<T, DIMS>(p, r[i], u[i], a, b, M[i], Ma, Mb);
-            }
+            r[i] = mobility_update<T, DIMS>(p, r[i], u[i], a, b, M[i], Ma, Mb);
         }
     }
 }
 
 // f'_s into out (X updated), the pseudospectral path's model evaluation
-template <typename T>
+template <typename T, class MD>
 __global__ __launch_bounds__(256) void k_sp_fprime(const T *__restrict__ rho, double *__restrict__ Xf,
-                                                   T *__restrict__ out, const SpModel *__restrict__ mp, int64_t bins) {
-    const SpModel &m = *mp;
+                                                   T *__restrict__ out, typename MD::M arg, int64_t bins) {
+    const auto &m = model_of(arg);
     SP_CELLS {
-        double rhos[kSpMaxSpecies], X[kSpMaxPatches], f[kSpMaxSpecies];
-        for(int s = 0; s < m.S; s++) rhos[s] = (double)rho[s * bins + i];
-        for(int q = 0; q < m.P; q++) X[q] = Xf[q * bins + i];
-        sp_fprime(m, rhos, X, f);
-        for(int q = 0; q < m.P; q++) Xf[q * bins + i] = X[q];
-        for(int s = 0; s < m.S; s++) out[s * bins + i] = (T)f[s];
+        double rhos[MD::S], X[MD::P], f[MD::S];
+        load_cell<MD>(m, rho, Xf, i, bins, rhos, X);
+        sp_fprime<MD>(m, rhos, X, f);
+        each_patch<MD>(m, [&](int q) { Xf[q * bins + i] = X[q]; });
+        each_species<MD>(m, [&](int s) { out[s * bins + i] = (T)f[s]; });
     }
 }
 
@@ -298,7 +452,8 @@ __global__ __launch_bounds__(256) void k_sp_mob(const T *__restrict__ rho, const
     SP_CELLS {
         double X[kSpMaxPatches];
         for(int q = 0; q < m.P; q++) X[q] = Xf[q * bins + i];
-        for(int s = 0; s < m.S; s++) out[s * bins + i] = sp_mobility(p, m, mob, s, (double)rho[s * bins + i], X);
+        for(int s = 0; s < m.S; s++)
+            out[s * bins + i] = sp_mobility<LargeModel>(p, m, mob, s, (double)rho[s * bins + i], X);
     }
 }
 #undef SP_CELLS
@@ -376,6 +531,51 @@ hipError_t by_precision(int precision, F &&f) {
 
 int grid_for(int64_t n) { return (int)std::min<int64_t>(kSpBlocks, (n + 255) / 256); }
 
+bool is_small(const SpModel &m) {
+    return m.model != CH_GENERIC_WERTHEIM || (m.S <= kSpSmall && m.P <= kSpSmall && m.n_unique == m.P);
+}
+
+SpSmallModel small_model(const SpModel &in) {
+    SpSmallModel m{};
+    m.model = in.model;
+    m.S = in.S;
+    m.P = in.P;
+    for(int i = 0; i < 3; i++) m.val[i] = in.val[i];
+    m.lh = in.lh;
+    m.sB2 = in.sB2;
+    m.sB3 = in.sB3;
+    m.dAA = in.dAA;
+    m.dBB = in.dBB;
+    m.rB2 = in.rB2;
+    m.d00 = in.d00;
+    m.d12 = in.d12;
+    for(int a = 0; a < kSpSmall; a++) {
+        m.k[a] = in.k[a];
+        for(int b = 0; b < kSpSmall; b++) {
+            m.pc[a][b] = in.pc[a][b];
+            m.B2[a][b] = in.B2[a][b];
+            m.dl[a][b] = in.delta[a][b];
+        }
+    }
+    return m;
+}
+
+// f(model tag, kernel argument): the model form with static sizes where it applies
+template <typename F>
+hipError_t by_model(const SpArgs &a, F &&f) {
+    const SpModel &m = *a.m_host;
+    if(!is_small(m)) return f(LargeModel{}, a.m);
+    const SpSmallModel sm = small_model(m);
+    if(m.model == CH_SALEH_WERTHEIM) return f(SalehModel{}, sm);
+    if(m.model == CH_RICCI_WERTHEIM) return f(RicciModel{}, sm);
+    switch(m.P) {
+    case 1: return f(SmallModel<1>{}, sm);
+    case 2: return f(SmallModel<2>{}, sm);
+    case 3: return f(SmallModel<3>{}, sm);
+    default: return f(SmallModel<4>{}, sm);
+    }
+}
+
 }  // namespace
 
 void sp_build_model(const ch_species_model &in, SpModel &m) {
@@ -404,6 +604,8 @@ void sp_build_model(const ch_species_model &in, SpModel &m) {
     for(int s = 0; s < m.S; s++)
         for(int q = 0; q < m.P; q++)
             if(m.pc[s][q] > 0) used[q] = 1;
+    for(int q = 0; q < m.P; q++)
+        for(int o = 0; o < m.P; o++) m.delta[q][o] = used[q] && used[o] && in.delta[q][o] > 0.0 ? in.delta[q][o] : 0.0;
     int nt = 0;
     for(int q = 0; q < m.P; q++) {
         if(!used[q]) continue;
@@ -426,8 +628,11 @@ hipError_t sp_warm(const SpArgs &a, hipStream_t s) {
     if(a.m_host->model != CH_GENERIC_WERTHEIM) return hipSuccess;
     return by_precision<1>(a.precision, [&](auto tag) {
         using T = decltype(tag);
-        hipLaunchKernelGGL((k_sp_warm<T>), dim3(grid_for(a.bins)), dim3(256), 0, s, (const T *)a.rho, a.X, a.m, a.bins);
-        return hipGetLastError();
+        return by_model(a, [&](auto md, const auto &arg) {
+            hipLaunchKernelGGL((k_sp_warm<T, decltype(md)>), dim3(grid_for(a.bins)), dim3(256), 0, s, (const T *)a.rho,
+                               a.X, arg, a.bins);
+            return hipGetLastError();
+        });
     });
 }
 
@@ -436,16 +641,20 @@ hipError_t sp_step_stencil(const SpArgs &a, int integrator, hipStream_t s) {
         using T = decltype(tag);
         const int g = grid_for(a.bins);
         const int mob = integrator == CH_EULER_MOBILITY ? a.mob_rule : -1;
-        auto go = [&](auto dims_tag) {
+        auto go = [&](auto dims_tag) -> hipError_t {
             constexpr int D = decltype(dims_tag)::value;
-            hipLaunchKernelGGL((k_sp_mu<T, D>), dim3(g), dim3(256), 0, s, (const T *)a.rho, a.X, (T *)a.mu, (T *)a.mob,
-                               a.p, a.m, a.bins, mob);
+            hipError_t e = by_model(a, [&](auto md, const auto &arg) {
+                hipLaunchKernelGGL((k_sp_mu<T, D, decltype(md)>), dim3(g), dim3(256), 0, s, (const T *)a.rho, a.X,
+                                   (T *)a.mu, (T *)a.mob, a.p, arg, a.bins, mob);
+                return hipGetLastError();
+            });
+            if(e != hipSuccess) return e;
             if(integrator == CH_EULER_MOBILITY)
-                hipLaunchKernelGGL((k_sp_update<T, D, true>), dim3(g), dim3(256), 0, s, (T *)a.rho, (const T *)a.mu,
-                                   (const T *)a.mob, a.p, a.m_host->S, a.bins);
+                hipLaunchKernelGGL((k_sp_update<T, D, true>), dim3(g, a.m_host->S), dim3(256), 0, s, (T *)a.rho,
+                                   (const T *)a.mu, (const T *)a.mob, a.p, a.bins);
             else
-                hipLaunchKernelGGL((k_sp_update<T, D, false>), dim3(g), dim3(256), 0, s, (T *)a.rho, (const T *)a.mu,
-                                   (const T *)a.mob, a.p, a.m_host->S, a.bins);
+                hipLaunchKernelGGL((k_sp_update<T, D, false>), dim3(g, a.m_host->S), dim3(256), 0, s, (T *)a.rho,
+                                   (const T *)a.mu, (const T *)a.mob, a.p, a.bins);
             return hipGetLastError();
         };
         if(a.p.dims == 1) return go(std::integral_constant<int, 1>{});
@@ -458,9 +667,11 @@ hipError_t sp_step_spectral(const SpArgs &a, const SpectralArgs &sa, hipStream_t
     return by_precision<1>(a.precision, [&](auto tag) -> hipError_t {
         using T = decltype(tag);
         const int S = a.m_host->S;
-        hipLaunchKernelGGL((k_sp_fprime<T>), dim3(grid_for(a.bins)), dim3(256), 0, s, (const T *)a.rho, a.X, (T *)a.mu,
-                           a.m, a.bins);
-        hipError_t e = hipGetLastError();
+        hipError_t e = by_model(a, [&](auto md, const auto &arg) {
+            hipLaunchKernelGGL((k_sp_fprime<T, decltype(md)>), dim3(grid_for(a.bins)), dim3(256), 0, s,
+                               (const T *)a.rho, a.X, (T *)a.mu, arg, a.bins);
+            return hipGetLastError();
+        });
         for(int sp = 0; sp < S && e == hipSuccess; sp++) {
             SpectralArgs b = sa;
             b.rho = (T *)a.rho + sp * a.bins;
