@@ -68,6 +68,7 @@ struct ch_sys {
     void *psm_spec[4] = {nullptr, nullptr, nullptr, nullptr};
     void *psm_field[3] = {nullptr, nullptr, nullptr};
     void *psm_vec[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};  // V, w, b, x, rhs, r, av
+    double *psm_max = nullptr;   // partial maxima of the mobility (N^(dims - 1) or kPsmParts)
     double *psm_dev = nullptr;   // kPsmParts partials, 4 scalars, Hcol, y
     double *psm_host = nullptr;  // pinned, kPsmParts doubles
     // pinned: mass and free energy written by the finalize kernel, the pair of
@@ -355,6 +356,7 @@ static void free_sys(ch_sys *s) {
     for(void *b : s->psm_vec)
         if(b) (void)hipFree(b);
     if(s->psm_dev) (void)hipFree(s->psm_dev);
+    if(s->psm_max) (void)hipFree(s->psm_max);
     for(void *b : {(void *)s->spm_dev, (void *)s->sp_X, s->sp_mu, s->sp_mob, s->sp_rho_hat, s->sp_spec[0], s->sp_spec[1]})
         if(b) (void)hipFree(b);
     delete s->spm_host;
@@ -429,6 +431,7 @@ extern "C" ch_status ch_sys_create(ch_ctx *ctx, const ch_desc *desc, ch_sys **ou
             ok = ok && alloc(&s->psm_vec[0], (size_t)(m + 1) * s->bins * s->elt);
             for(int i = 1; i < 7; i++) ok = ok && alloc(&s->psm_vec[i], s->bins * s->elt);
         }
+        ok = ok && alloc((void **)&s->psm_max, sizeof(double) * std::max<int64_t>(chd::kPsmParts, s->bins / N));
         ok = ok && alloc((void **)&s->psm_dev, sizeof(double) * (chd::kPsmParts + 4 + 2 * (m + 2))) &&
              hipHostMalloc((void **)&s->psm_host, sizeof(double) * std::max(chd::kPsmParts, m + 2)) == hipSuccess;
     }
@@ -838,6 +841,7 @@ static chd::PsmArgs psm_args(ch_sys *s) {
     B.r = s->psm_vec[5];
     B.av = s->psm_vec[6];
     B.fuse = s->psm_fuse;
+    B.max_parts = s->psm_max;
     return B;
 }
 
@@ -855,26 +859,18 @@ static ch_status evolve_psm(ch_sys *s, int64_t nsteps) {
         }
         return CH_OK;
     }
+    auto chain = [&](int64_t n) { return chd::psm_steps_simple(B, n, c->stream); };
     const int G = s->graph_steps;
     if(G > 0 && nsteps >= G) {
         if(!s->gexec[0]) {
-            hipGraph_t graph;
-            HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-            hipError_t e = hipSuccess;
-            for(int i = 0; i < G && e == hipSuccess; i++) e = chd::psm_step_simple(B, c->stream);
-            hipError_t e2 = hipStreamEndCapture(c->stream, &graph);
-            if(e != hipSuccess) return fail(c, CH_EHIP, "step launch during capture failed: %s", hipGetErrorString(e));
-            if(e2 != hipSuccess) return fail(c, CH_EHIP, "hipStreamEndCapture failed: %s", hipGetErrorString(e2));
-            e = hipGraphInstantiate(&s->gexec[0], graph, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(graph);
-            if(e != hipSuccess) return fail(c, CH_EHIP, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
+            ch_status st = capture(c, s->gexec[0], [&] { return chain(G); });
+            if(st != CH_OK) return st;
         }
         const int64_t reps = nsteps / G;
         for(int64_t r = 0; r < reps; r++) HIPCHK(c, hipGraphLaunch(s->gexec[0], c->stream));
         nsteps -= reps * G;
     }
-    for(int64_t i = 0; i < nsteps; i++) HIPCHK(c, chd::psm_step_simple(B, c->stream));
-    return CH_OK;
+    return replay_recurring(s, nsteps, chain);
 }
 
 extern "C" int32_t ch_sys_gmres_iterations(const ch_sys *s) { return s ? s->gmres_iters : 0; }

@@ -66,6 +66,11 @@ hipError_t ps_steps_tape(const SpectralArgs &a, hipStream_t s, int64_t nsteps, v
 // fprime) into spec; c2r of spec (overwritten) into out
 hipError_t spec_r2c(const SpectralArgs &a, const void *real_in, void *spec_out, bool fprime, hipStream_t s);
 hipError_t spec_c2r(const SpectralArgs &a, void *spec, void *real_out, hipStream_t s);
+// single passes of those transforms: the x pass alone, and the y pass of a 3D
+// half spectrum in place
+hipError_t spec_x_forward(const SpectralArgs &a, const void *real_in, void *spec_out, bool fprime, hipStream_t s);
+hipError_t spec_x_inverse(const SpectralArgs &a, const void *spec, void *real_out, hipStream_t s);
+hipError_t spec_y_pass(const SpectralArgs &a, void *spec, bool inverse, hipStream_t s);
 // pseudospectral_mobility: divh = sum_d (i k_d) deal r2c(w c2r((i k_d) deal src) / N^d),
 // w = M - M0 (sub, M0 = *M0p) or M, with the element-wise work inside the
 // transform passes; hipErrorNotSupported outside 2D N = 1024, 2048
@@ -101,10 +106,15 @@ struct PsmArgs {
     void *w, *b, *x, *rhs, *r, *av;
     double *Hcol, *ydev;          // restart + 2 doubles each (device)
     double *host_partials;        // pinned host memory, kPsmParts doubles
-    bool fuse;                    // divergence term through psm_div_fused where it applies
+    bool fuse;                    // splitting chain and divergence term through the fused passes
+    double *max_parts;            // N^(dims - 1) (at least kPsmParts) partial maxima of the mobility
 };
-// one splitting step, asynchronous (capturable)
-hipError_t psm_step_simple(const PsmArgs &B, hipStream_t s);
+// nsteps splitting steps, asynchronous (capturable)
+hipError_t psm_steps_simple(const PsmArgs &B, int64_t nsteps, hipStream_t s);
+// the same in 2D and 3D as fused line passes (psm_pass.hip)
+hipError_t psm_chain(const PsmArgs &B, int64_t nsteps, hipStream_t s);
+// the mobility of rho into B.mob, its nparts (<= kPsmParts) partial maxima into `parts`
+hipError_t psm_mobility(const PsmArgs &B, double *parts, int &nparts, hipStream_t s);
 // one GMRES step, synchronous; iters = GMRES iterations
 hipError_t psm_step_full(const PsmArgs &B, hipStream_t s, int &iters);
 

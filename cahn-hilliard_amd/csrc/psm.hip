@@ -11,7 +11,9 @@
 //   rho_hat = (rho_hat + dt div_hat - dt M0 q^2 (f_hat - S rho_hat))
 //             / (1 + dt M0 (S q^2 + 2k q^4));   rho = c2r(rho_hat) / N^d
 // Everything stays on the device (M0 included), so a chain of steps is
-// captured into a graph like the other integrators.
+// captured into a graph like the other integrators.  In 2D and 3D the chain
+// runs as fused line passes (psm_pass.hip); 1D, and CH_PSM_FUSE=0, as the
+// element-wise kernels below around whole transforms.
 //
 // Full scheme (_evolve_full, :303-404): A x = b with
 //   A x = x - dt div(M grad((S - 2k lap) x)),  b = rho + dt div(M grad(f' - S rho)),
@@ -297,12 +299,12 @@ struct Ops {
     hipError_t r2c(const void *in, void *out, bool fprime = false) { return spec_r2c(B.a, in, out, fprime, s); }
     hipError_t c2r(void *in, void *out) { return spec_c2r(B.a, in, out, s); }
 
-    // M = mobility(rho) into B.mob and M0 into B.scal[0]
-    hipError_t mobility_and_m0() {
+    // M = mobility(rho) into B.mob, its grid_f partial maxima into `parts`
+    void mobility_field(double *parts) {
         auto go = [&](auto tag) {
             constexpr int MOB = decltype(tag)::value;
             hipLaunchKernelGGL((k_mob_max<T, MOB>), dim3(grid_f), dim3(256), 0, s, (const T *)B.a.rho, f(B.mob), p(),
-                               bins, B.partials);
+                               bins, parts);
         };
         switch(B.mob_rule) {
         case CH_MOB_CONSTANT: go(std::integral_constant<int, CH_MOB_CONSTANT>{}); break;
@@ -310,6 +312,10 @@ struct Ops {
         case CH_MOB_LINEAR: go(std::integral_constant<int, CH_MOB_LINEAR>{}); break;
         default: go(std::integral_constant<int, CH_MOB_FREE_ENERGY>{}); break;
         }
+    }
+    // M = mobility(rho) into B.mob and M0 into B.scal[0]
+    hipError_t mobility_and_m0() {
+        mobility_field(B.partials);
         hipLaunchKernelGGL(k_m0_final, dim3(1), dim3(256), 0, s, B.partials, grid_f, B.scal);
         return hipGetLastError();
     }
@@ -348,6 +354,15 @@ struct Ops {
                            (const C2<T> *)B.divh, c(B.muh), p(), hat, B.scal);
         e = hipGetLastError();
         if(e == hipSuccess) e = c2r(B.muh, B.a.rho);
+        return e;
+    }
+
+    hipError_t steps_simple(int64_t nsteps) {
+        hipError_t e = hipSuccess;
+        if(B.fuse && p().dims >= 2) {
+            return nsteps < 1 ? e : psm_chain(B, nsteps, s);
+        }
+        for(int64_t i = 0; i < nsteps && e == hipSuccess; i++) e = step_simple();
         return e;
     }
 
@@ -516,9 +531,19 @@ struct Ops {
 
 }  // namespace
 
-hipError_t psm_step_simple(const PsmArgs &B, hipStream_t s) {
-    if(B.a.precision == CH_FP64) return Ops<double>(B, s).step_simple();
-    return Ops<float>(B, s).step_simple();
+hipError_t psm_steps_simple(const PsmArgs &B, int64_t nsteps, hipStream_t s) {
+    if(B.a.precision == CH_FP64) return Ops<double>(B, s).steps_simple(nsteps);
+    return Ops<float>(B, s).steps_simple(nsteps);
+}
+
+hipError_t psm_mobility(const PsmArgs &B, double *parts, int &nparts, hipStream_t s) {
+    auto go = [&](auto tag) {
+        Ops<decltype(tag)> ops(B, s);
+        nparts = ops.grid_f;
+        ops.mobility_field(parts);
+        return hipGetLastError();
+    };
+    return B.a.precision == CH_FP64 ? go(double{}) : go(float{});
 }
 
 hipError_t psm_step_full(const PsmArgs &B, hipStream_t s, int &iters) {
