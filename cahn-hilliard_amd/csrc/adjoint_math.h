@@ -13,6 +13,12 @@ __device__ __forceinline__ double fsecond(const Params &p, double r) {
         return -p.eps + 3.0 * r * r;
     }
     else {
+        if(r > 0x1p-1000 && !(r < p.reg)) {
+            // valence X' / X = -valence c X / (2 c rho X + 1): one reciprocal of
+            // that sum and one of rho (dfprime_ddelta shares X and the first)
+            const double c = 0.5 * p.tvd, X = wertheim_X_pos(p, r), q = recip_newton(2.0 * c * r * X + 1.0);
+            return 2 * p.B2 + recip_newton(r) - p.valence * (c * X * q);
+        }
         double d = 2 * p.B2 + ((r < p.reg) ? 1.0 / p.reg : 1.0 / r);
         if(r > 0.) {
             const double c = 0.5 * p.tvd, X = wertheim_X(p, r);
@@ -31,8 +37,8 @@ __device__ __forceinline__ double dfprime_ddelta(const Params &p, double r) {
     }
     else {
         if(!(r > 0.)) return 0.0;
-        const double c = 0.5 * p.tvd, X = wertheim_X(p, r);
-        return -(double)p.valence * p.valence * r * X / (2.0 * c * r * X + 1.0);
+        const double c = 0.5 * p.tvd, X = wertheim_X_pos(p, r), q = recip_newton(2.0 * c * r * X + 1.0);
+        return -(double)p.valence * p.valence * r * X * q;
     }
 }
 
@@ -68,11 +74,12 @@ __device__ __forceinline__ MobDeriv<MOB> mob_deriv(const Params &p, double r) {
         m.ddelta = p.M * r * v * Xv1 * (-v * r * X * X / den);
     }
     else if constexpr(MOB == CH_MOB_REGULARISED) {
-        m.hat = r / (r + p.rho_min);
-        m.drho = p.M * p.rho_min / ((r + p.rho_min) * (r + p.rho_min));
+        const double q = 1.0 / (r + p.rho_min);
+        m.hat = r * q;
+        m.drho = p.M * p.rho_min * q * q;
     }
     else if constexpr(MOB == CH_MOB_LINEAR) {
-        m.hat = r / p.rho_ref;
+        m.hat = r * (1.0 / p.rho_ref);
         m.drho = p.M / p.rho_ref;
     }
     return m;

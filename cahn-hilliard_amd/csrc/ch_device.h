@@ -44,6 +44,20 @@ struct Params {
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
+// a b + c for a literal c, read from a scalar register pair: the compiler's own
+// choice is a two-instruction copy of c into vector registers for every term of
+// a polynomial (a multiply-accumulate overwrites its addend), which makes each
+// term cost three vector instructions in place of one
+__device__ __forceinline__ double fma_const(double a, double b, double c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c));
+    return r;
+#else
+    return __builtin_fma(a, b, c);
+#endif
+}
+
 // ---------------------------------------------------------------- models
 // Landau: f' = -eps psi + psi^3 (src/models/Landau.cpp:46-52), evaluated in T.
 // SimpleWertheim: f' = 2 B2 rho + ln rho (or the linear branch below
@@ -59,8 +73,7 @@ __device__ __forceinline__ float fma_t(float a, float b, float c) { return __bui
 // exponent) plus the rest of its value.  Within 2 ulp (worst near m = 1) in
 // some 30 instructions, where the library log spends about 100; zero,
 // negative, infinite and NaN arguments go to log().
-__device__ __forceinline__ double log_series(double x) {
-    if(!(x > 0.0) || x == __builtin_inf()) return log(x);
+__device__ __forceinline__ double log_series_pos(double x) {  // 0 < x < inf
     double m = __builtin_amdgcn_frexp_mant(x);  // [0.5, 1), denormals included
     int e = __builtin_amdgcn_frexp_exp(x);
     if(m < 0.70710678118654752440) {
@@ -75,15 +88,15 @@ __device__ __forceinline__ double log_series(double x) {
     sv = __builtin_fma(__builtin_fma(-d, sv, f), r, sv);
     const double t = sv * sv;
     double q = 1.0 / 21.0;
-    q = __builtin_fma(q, t, 1.0 / 19.0);
-    q = __builtin_fma(q, t, 1.0 / 17.0);
-    q = __builtin_fma(q, t, 1.0 / 15.0);
-    q = __builtin_fma(q, t, 1.0 / 13.0);
-    q = __builtin_fma(q, t, 1.0 / 11.0);
-    q = __builtin_fma(q, t, 1.0 / 9.0);
-    q = __builtin_fma(q, t, 1.0 / 7.0);
-    q = __builtin_fma(q, t, 1.0 / 5.0);
-    q = __builtin_fma(q, t, 1.0 / 3.0);
+    q = fma_const(q, t, 1.0 / 19.0);
+    q = fma_const(q, t, 1.0 / 17.0);
+    q = fma_const(q, t, 1.0 / 15.0);
+    q = fma_const(q, t, 1.0 / 13.0);
+    q = fma_const(q, t, 1.0 / 11.0);
+    q = fma_const(q, t, 1.0 / 9.0);
+    q = fma_const(q, t, 1.0 / 7.0);
+    q = fma_const(q, t, 1.0 / 5.0);
+    q = fma_const(q, t, 1.0 / 3.0);
     const double u = 2.0 * sv;
     const double lm = __builtin_fma(u * t, q, u);
     const double ed = (double)e;
@@ -91,8 +104,41 @@ __device__ __forceinline__ double log_series(double x) {
     return __builtin_fma(ed, ln2_head, __builtin_fma(ed, ln2_rest, lm));
 }
 
+__device__ __forceinline__ double log_series(double x) {
+    if(!(x > 0.0) || x == __builtin_inf()) return log(x);
+    return log_series_pos(x);
+}
+
 __device__ __forceinline__ double wertheim_X(const Params &p, double r) {
     return (-1.0 + sqrt(1.0 + 2.0 * p.tvd * r)) / (p.tvd * r);
+}
+
+// 1 / d for d normal and finite: the hardware's reciprocal and two Newton steps,
+// within 1 ulp (no scaling for the extremes of the range)
+__device__ __forceinline__ double recip_newton(double d) {
+#pragma clang fp contract(off)
+    const double q = __builtin_amdgcn_rcp(d);
+    const double r = __builtin_fma(__builtin_fma(-d, q, 1.0), q, q);
+    return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+}
+
+// X(rho) for rho > 0 in the stepping kernels, as 2 / (1 + sqrt(1 + 2 tvd rho)) (the
+// same root without the difference): the square root of an argument above 1 by
+// one Goldschmidt step and a residual correction on the hardware's reciprocal
+// root, the quotient by the hardware's reciprocal and two Newton steps.  17
+// operations where the IEEE square root and division, with their scaling for
+// every exponent, take about 40; within 2.5e-16 relative (a host restatement
+// with seeds off by 1e-7, against long double, 20 M arguments 1e-12 < tvd rho < 1e18).
+__device__ __forceinline__ double wertheim_X_pos(const Params &p, double r) {
+#pragma clang fp contract(off)
+    const double x = __builtin_fma(2.0 * p.tvd, r, 1.0);
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return 2.0 * recip_newton(1.0 + g);
 }
 
 template <typename T, int MODEL>
@@ -104,21 +150,23 @@ __device__ __forceinline__ T fprime(const Params &p, T r) {
         return r * fma_t(r, r, -(T)p.eps);
     }
     else {
+        // ln rho + valence ln X = ln(rho X^valence): one logarithm.  One test
+        // covers everything else (rho below the regularisation, not positive, or
+        // a product out of range), so a wave of ordinary densities runs straight
         const double rd = (double)r;
-        double d = 2 * p.B2 * rd;
-        if(rd < p.reg) {
-            d += p.log_reg + (rd - p.reg) / p.reg;
-            if(rd > 0.) d += p.valence * log_series(wertheim_X(p, rd));
-        }
-        else if(rd > 0.) {
-            // ln rho + valence ln X = ln(rho X^valence): one logarithm
-            const double X = wertheim_X(p, rd);
-            double xv = rd;
-            for(int i = 0; i < p.valence; i++) xv *= X;
-            d += log_series(xv);
-        }
-        else {
-            d += log(rd);
+        const double X = wertheim_X_pos(p, rd);
+        double xv = rd;
+        for(int i = 0; i < p.valence; i++) xv *= X;
+        double d = 2 * p.B2 * rd + log_series_pos(xv);
+        if(__builtin_expect(!(rd >= p.reg && rd > 0. && xv > 0. && xv < __builtin_inf()), 0)) {
+            d = 2 * p.B2 * rd;
+            if(rd < p.reg) {
+                d += p.log_reg + (rd - p.reg) / p.reg;
+                if(rd > 0.) d += p.valence * log_series_pos(X);
+            }
+            else {
+                d += log(rd > 0. ? xv : rd);
+            }
         }
         return (T)d;
     }
@@ -150,6 +198,17 @@ __device__ __forceinline__ double bulk(const Params &p, double r) {
     }
 }
 
+// a / b for a divisor b that all threads share: 1 / b once per thread (hoisted
+// out of its loop over cells), then the quotient and its residual correction --
+// the IEEE quotient's bits (Markstein: exact unless b's significand is all
+// ones) in 3 operations per cell for 14
+template <typename T>
+__device__ __forceinline__ T div_uniform(T a, T b) {
+#pragma clang fp contract(off)
+    const T r = (T)1 / b, q = a * r;
+    return fma_t(fma_t(-q, b, a), r, q);
+}
+
 // ---------------------------------------------------------------- mobility
 // constant (ConstantMobility.h:19-23), free_energy (FreeEnergyMobility.h:25-34
 // -> SimpleWertheim.cpp:104-111), regularised (RegularisedMobility.h:26-33),
@@ -161,6 +220,13 @@ __device__ __forceinline__ T mobility(const Params &p, T r) {
     }
     else if constexpr(MOB == CH_MOB_FREE_ENERGY) {
         double rd = (double)r;
+        if(rd > 0.) {
+            // X^valence by products: 4 to 10 operations for pow's 200
+            const double X = wertheim_X_pos(p, rd);
+            double Xv = X;
+            for(int i = 1; i < p.valence; i++) Xv *= X;
+            return (T)(rd * (p.M * Xv));
+        }
         double X = wertheim_X(p, rd);
         double D = p.M * pow(X, (double)p.valence);
         return (T)(rd * D);
@@ -169,7 +235,7 @@ __device__ __forceinline__ T mobility(const Params &p, T r) {
         return (T)p.M * r / (r + (T)p.rho_min);
     }
     else {
-        return (T)p.M * r / (T)p.rho_ref;
+        return div_uniform((T)p.M * r, (T)p.rho_ref);
     }
 }
 

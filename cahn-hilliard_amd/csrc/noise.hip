@@ -59,19 +59,19 @@ __device__ __forceinline__ void sincos_2pi(double u, double &sn, double &cs) {
     const double r = __builtin_fma(f, 0.7853981633974483, f * 3.061616997868383e-17);
     const double t = r * r;
     double s = -1.0 / 6227020800.0;  // -1/13!
-    s = __builtin_fma(s, t, 1.0 / 39916800.0);
-    s = __builtin_fma(s, t, -1.0 / 362880.0);
-    s = __builtin_fma(s, t, 1.0 / 5040.0);
-    s = __builtin_fma(s, t, -1.0 / 120.0);
-    s = __builtin_fma(s, t, 1.0 / 6.0);
+    s = fma_const(s, t, 1.0 / 39916800.0);
+    s = fma_const(s, t, -1.0 / 362880.0);
+    s = fma_const(s, t, 1.0 / 5040.0);
+    s = fma_const(s, t, -1.0 / 120.0);
+    s = fma_const(s, t, 1.0 / 6.0);
     const double sr = __builtin_fma(-r * t, s, r);  // r - r^3 (1/3! - r^2/5! + ...)
     double c = 1.0 / 87178291200.0;                 // 1/14!
-    c = __builtin_fma(c, t, -1.0 / 479001600.0);
-    c = __builtin_fma(c, t, 1.0 / 3628800.0);
-    c = __builtin_fma(c, t, -1.0 / 40320.0);
-    c = __builtin_fma(c, t, 1.0 / 720.0);
-    c = __builtin_fma(c, t, -1.0 / 24.0);
-    c = __builtin_fma(c, t, 0.5);
+    c = fma_const(c, t, -1.0 / 479001600.0);
+    c = fma_const(c, t, 1.0 / 3628800.0);
+    c = fma_const(c, t, -1.0 / 40320.0);
+    c = fma_const(c, t, 1.0 / 720.0);
+    c = fma_const(c, t, -1.0 / 24.0);
+    c = fma_const(c, t, 0.5);
     const double cr = __builtin_fma(-t, c, 1.0);  // 1 - r^2 (1/2! - r^2/4! + ...)
     constexpr double S1 = 0.3826834323650898, C1 = 0.9238795325112867;  // sin, cos of pi/8
     const bool swap = k == 1 || k == 2 || k == 5 || k == 6;
@@ -94,7 +94,7 @@ __device__ __forceinline__ void cell_normals(uint64_t seed, uint32_t cell, uint6
         if constexpr(sizeof(T) == 8) {
             const double u1 = ((double)w[2 * h] + 0.5) * 0x1p-32;
             const double u2 = ((double)w[2 * h + 1] + 0.5) * 0x1p-32;
-            const double r = sqrt(-2.0 * log_series(u1));
+            const double r = sqrt(-2.0 * log_series_pos(u1));
             double sn, cs;
             sincos_2pi(u2, sn, cs);
             eta[2 * h] = r * cs;

@@ -64,14 +64,6 @@ __device__ __forceinline__ double saleh_log_X(const SpSmallModel &m, const doubl
     return rho_factor >= 0 ? log_series(X) : 0.0;
 }
 
-// 1 / d for d in [1, 2^100): the hardware reciprocal and two Newton steps, within
-// 1 ulp in five dependent operations where the IEEE division takes about ten
-__device__ __forceinline__ double recip(double d) {
-    double r = __builtin_amdgcn_rcp(d);
-    r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
-    return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
-}
-
 // generic_update_X's sweeps, on X_p = 1 / (1 + sum_q a_pq X_q)
 template <int P, bool SHORT>
 __device__ __forceinline__ void small_sweeps(const double (&a)[P][P], double (&X)[P]) {
@@ -84,7 +76,7 @@ __device__ __forceinline__ void small_sweeps(const double (&a)[P][P], double (&X
             double sum = 1.0;
 #pragma unroll
             for(int q = 0; q < P; q++) sum = __builtin_fma(a[p][q], X[q], sum);
-            const double new_X = SHORT ? recip(sum) : 1.0 / sum;
+            const double new_X = SHORT ? recip_newton(sum) : 1.0 / sum;
             const double d = fabs(new_X - X[p]);
             max_delta = (max_delta < d) ? d : max_delta;
             X[p] = new_X;
