@@ -33,6 +33,12 @@ bool adjoint_split3d_ok(const Params &p, int mob);
 int adjoint_split3d_blocks(const Params &p);
 hipError_t adjoint_split3d(const Params &p, int precision, int model, int mob, const void *lam_in, void *lam_out,
                            const void *psi, void *const work[4], bool have_mu, double *gacc, hipStream_t s);
+// the 3D step in one launch marching along z (Params::tile3d >= 4, N >= 32), and
+// whether it is the faster form
+inline bool march3d_ok(const Params &p) { return p.tile3d >= 4 && p.N >= 32; }
+bool march3d_better(const Params &p, int precision, int integrator, int model, int mob);
+hipError_t stencil_march3d(const Params &p, int precision, int integrator, int model, int mob, const void *in,
+                           void *out, hipStream_t s);
 inline int stencil_max_k(int dims, int N) { return (dims == 2 && N >= 64) ? 8 : 1; }
 // one euler_mobility step with conserved noise (noise.hip), in -> out; the
 // step index is *step_base + step_off.  noise_step_advance adds n to *step_base.

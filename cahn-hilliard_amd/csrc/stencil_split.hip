@@ -319,7 +319,7 @@ hipError_t split3d_mu(const Params &p, int precision, int integrator, int model,
 }
 
 bool adjoint_split3d_ok(const Params &p, int mob) {
-    return p.tile3d == 3 && split3d_ok(p, CH_EULER_MOBILITY, mob) && p.N % kAdjZNu == 0;
+    return (p.tile3d == 3 || p.tile3d == 5) && split3d_ok(p, CH_EULER_MOBILITY, mob) && p.N % kAdjZNu == 0;
 }
 
 int adjoint_split3d_blocks(const Params &p) { return (int)(((int64_t)1 << (3 * p.log2N)) / (256 * kAdjZUpd)); }
