@@ -20,6 +20,7 @@
 // built on the host from exact integer indices (rounded once for FP32).
 #include "line_fft.h"
 #include "psm_ops.h"
+#include "spec_plane.h"
 
 namespace chd {
 
@@ -815,6 +816,14 @@ static hipError_t ps_chain_t(const SpectralArgs &a, hipStream_t s, int64_t nstep
     const bool landau = a.model == CH_LANDAU;
     const size_t bins = (size_t)rows * N;
     const bool rhl = a.rh_lines && dims == 2 && (LOG2N == 10 || LOG2N == 11);
+    const bool planes = dims == 3 && plane_len<T>(LOG2N);
+    if constexpr(plane_len<T>(LOG2N)) {
+        if(planes && init) {
+            launch_plane<T, CH_LANDAU, LOG2N, PLANE_R2C>(W, tw2, p, rho, s);
+            pass_z<T, 0, LOG2N>(L, W, RH, tw2, p, lines, s, RH);
+            return hipGetLastError();
+        }
+    }
     if(init) {
         launch_xfwd<T, CH_LANDAU, false, LX>(rho, dims == 1 ? RH : W, tw2, p, rows, L.rs, L.ks, s);
         if(dims == 2) pass_y<T, 0, LOG2N>(L, W, RH, tw2, p, lines, s, RH, rhl);
@@ -825,9 +834,13 @@ static hipError_t ps_chain_t(const SpectralArgs &a, hipStream_t s, int64_t nstep
         return hipGetLastError();
     }
     if(nsteps < 1) return hipSuccess;
-    if(landau)
+    if constexpr(plane_len<T>(LOG2N)) {
+        if(planes && landau) launch_plane<T, CH_LANDAU, LOG2N, PLANE_FPRIME>(W, tw2, p, rho, s);
+        if(planes && !landau) launch_plane<T, CH_SIMPLE_WERTHEIM, LOG2N, PLANE_FPRIME>(W, tw2, p, rho, s);
+    }
+    if(!planes && landau)
         launch_xfwd<T, CH_LANDAU, true, LX>(rho, W, tw2, p, rows, L.rs, L.ks, s);
-    else
+    else if(!planes)
         launch_xfwd<T, CH_SIMPLE_WERTHEIM, true, LX>(rho, W, tw2, p, rows, L.rs, L.ks, s);
     for(int64_t t = 0; t < nsteps; t++) {
         if(dims == 1) {
@@ -837,20 +850,35 @@ static hipError_t ps_chain_t(const SpectralArgs &a, hipStream_t s, int64_t nstep
             pass_y<T, 2, LOG2N>(L, W, RH, tw2, p, lines, s, nullptr, rhl);
         }
         else {
-            // y forward (line l: plane l / Nh, column l % Nh), the fused z pass, y inverse
-            pass_y<T, 0, LOG2N>(L, W, RH, tw2, p, lines, s);
+            // y forward (line l: plane l / Nh, column l % Nh), the fused z pass, y
+            // inverse; with the plane passes the y passes belong to those
+            if(!planes) pass_y<T, 0, LOG2N>(L, W, RH, tw2, p, lines, s);
             pass_z<T, 2, LOG2N>(L, W, RH, tw2, p, lines, s);
-            pass_y<T, 1, LOG2N>(L, W, RH, tw2, p, lines, s);
+            if(!planes) pass_y<T, 1, LOG2N>(L, W, RH, tw2, p, lines, s);
         }
         if(t + 1 < nsteps) {
             T *ro = tape ? tape + (size_t)(t + 1) * bins : nullptr;
+            if constexpr(plane_len<T>(LOG2N)) {
+                if(planes) {
+                    if(landau) launch_plane<T, CH_LANDAU, LOG2N, PLANE_BOTH>(W, tw2, p, ro, s);
+                    else launch_plane<T, CH_SIMPLE_WERTHEIM, LOG2N, PLANE_BOTH>(W, tw2, p, ro, s);
+                    continue;
+                }
+            }
             if(landau)
                 launch_xrow<T, CH_LANDAU, LX>(W, tw2, p, rows, L.rs, L.ks, ro, s);
             else
                 launch_xrow<T, CH_SIMPLE_WERTHEIM, LX>(W, tw2, p, rows, L.rs, L.ks, ro, s);
         }
     }
-    launch_xinv<T, LX>(W, tape ? tape + (size_t)nsteps * bins : rho, tw2, p, rows, L.rs, L.ks, s);
+    T *last = tape ? tape + (size_t)nsteps * bins : rho;
+    if constexpr(plane_len<T>(LOG2N)) {
+        if(planes) {
+            launch_plane<T, CH_LANDAU, LOG2N, PLANE_C2R>(W, tw2, p, last, s);
+            return hipGetLastError();
+        }
+    }
+    launch_xinv<T, LX>(W, last, tw2, p, rows, L.rs, L.ks, s);
     return hipGetLastError();
 }
 
