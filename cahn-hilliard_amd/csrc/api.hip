@@ -269,9 +269,9 @@ static chd::Params make_params(const ch_desc *d) {
     if(split) p.tile3d = 3;
     if(d->dims == 3 && chd::march3d_better(p, d->precision, d->integrator, d->model, d->mobility)) p.tile3d = split ? 5 : 4;
     p.adj_tile3d = 1;
-    // noise step: 64 x 32 (2D) and 16 x 8 x 8 (3D) tiles of 512 threads measured
-    // 10 % and 30 % faster than 64 x 16 and 8 x 8 x 8 with 256
-    p.noise_tile = 2;
+    // noise step tiles: 64 x 32 in 2D from N = 1024, else 64 x 16 (twice the
+    // blocks) and 8 x 8 x 8 in 3D, all with 512 threads (figures in noise.hip)
+    p.noise_tile = d->dims == 2 && d->N >= 1024 ? 2 : 1;
     p.S = d->S;
     double bins = std::pow((double)d->N, d->dims);
     p.vbin_over_bins = d->dx * d->dx * d->dx / bins;

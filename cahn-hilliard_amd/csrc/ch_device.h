@@ -21,7 +21,7 @@ struct Params {
     int adj_cfg;           // region shape of the 2D wave adjoint (0, 3, 4 or 5)
     int tile3d;            // 3D forward step: LDS tile 0: 16x8x8 / 256 threads, 1: the same / 512, 2: 16x16x4 / 512; 3: two launches (stencil_split.hip); 4, 5: one launch marching along z (stencil_march.hip; 5: the reverse step in two launches)
     int adj_tile3d;        // 3D tile of the euler_mobility adjoint (0: 16x4x4 / 256, 1 (default): 16x8x4 / 512, 2: 16x8x8 / 512)
-    int noise_tile;        // tile of the noise step (0: 2D 64x16, 3D 8x8x8 / 256 threads; 1: the same / 512; 2 (default): 2D 64x32, 3D 16x8x8 / 512)
+    int noise_tile;        // tile of the noise step (0: 2D 64x16, 3D 8x8x8 / 256 threads; 1 (default): the same / 512; 2 (default for 2D N >= 1024): 2D 64x32, 3D 16x8x8 / 512)
     double eps;            // Landau epsilon
     double B2, reg, log_reg, tvd;   // SimpleWertheim: tvd = 2 valence delta
     double M, rho_min, rho_ref;     // mobility
@@ -122,23 +122,28 @@ __device__ __forceinline__ double recip_newton(double d) {
     return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
 }
 
+// sqrt(x) for x > 0, normal, well inside the exponent range: one Goldschmidt step
+// and a residual correction on the hardware's reciprocal root (within 1 ulp;
+// the IEEE root scales its argument and corrects twice)
+__device__ __forceinline__ double sqrt_normal(double x) {
+#pragma clang fp contract(off)
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
 // X(rho) for rho > 0 in the stepping kernels, as 2 / (1 + sqrt(1 + 2 tvd rho)) (the
-// same root without the difference): the square root of an argument above 1 by
-// one Goldschmidt step and a residual correction on the hardware's reciprocal
-// root, the quotient by the hardware's reciprocal and two Newton steps.  17
+// same root without the difference), with the short root and reciprocal: 17
 // operations where the IEEE square root and division, with their scaling for
 // every exponent, take about 40; within 2.5e-16 relative (a host restatement
 // with seeds off by 1e-7, against long double, 20 M arguments 1e-12 < tvd rho < 1e18).
 __device__ __forceinline__ double wertheim_X_pos(const Params &p, double r) {
 #pragma clang fp contract(off)
     const double x = __builtin_fma(2.0 * p.tvd, r, 1.0);
-    const double y = __builtin_amdgcn_rsq(x);
-    double g = x * y, h = 0.5 * y;
-    const double e = __builtin_fma(-h, g, 0.5);
-    g = __builtin_fma(g, e, g);
-    h = __builtin_fma(h, e, h);
-    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-    return 2.0 * recip_newton(1.0 + g);
+    return 2.0 * recip_newton(1.0 + sqrt_normal(x));
 }
 
 template <typename T, int MODEL>

@@ -37,9 +37,10 @@ __device__ __forceinline__ uint4 philox4x32_10(uint4 c, uint32_t k0, uint32_t k1
             k0 += W0;
             k1 += W1;
         }
-        const uint32_t hi0 = __umulhi(M0, c.x), lo0 = M0 * c.x;
-        const uint32_t hi1 = __umulhi(M1, c.z), lo1 = M1 * c.z;
-        c = uint4{hi1 ^ c.y ^ k0, lo1, hi0 ^ c.w ^ k1, lo0};
+        // one 64-bit multiply-add each, where the halves apart are two
+        // quarter-rate products
+        const uint64_t p0 = (uint64_t)M0 * c.x, p1 = (uint64_t)M1 * c.z;
+        c = uint4{(uint32_t)(p1 >> 32) ^ c.y ^ k0, (uint32_t)p1, (uint32_t)(p0 >> 32) ^ c.w ^ k1, (uint32_t)p0};
     }
     return c;
 }
@@ -82,6 +83,29 @@ __device__ __forceinline__ void sincos_2pi(double u, double &sn, double &cs) {
     cs = __builtin_fma(ck, cr, -(sk * sr));
 }
 
+// the same in FP32: r = f pi / 4 with f exact, series through r^7 and r^8 (first
+// omitted terms below 3e-9), where sincosf of the rounded product 2 pi u reduces
+// a general argument
+__device__ __forceinline__ void sincos_2pi(float u, float &sn, float &cs) {
+#pragma clang fp contract(off)
+    const float v = 8.0f * u;
+    const int k = (int)v;
+    const float r = ((v - (float)k) - 0.5f) * 0.78539816339744830962f;
+    const float t = r * r;
+    float s = fma_t(fma_t(-1.0f / 5040.0f, t, 1.0f / 120.0f), t, -1.0f / 6.0f);
+    const float sr = fma_t(r * t, s, r);
+    float c = fma_t(fma_t(fma_t(1.0f / 40320.0f, t, -1.0f / 720.0f), t, 1.0f / 24.0f), t, -0.5f);
+    const float cr = fma_t(t, c, 1.0f);
+    constexpr float S1 = 0.38268343236508977173f, C1 = 0.92387953251128675613f;  // sin, cos of pi/8
+    const int o = k & 7;  // u = 1 after rounding: octant 8
+    const bool swap = o == 1 || o == 2 || o == 5 || o == 6;
+    float sk = swap ? C1 : S1, ck = swap ? S1 : C1;
+    if(o >= 4) sk = -sk;
+    if(o >= 2 && o <= 5) ck = -ck;
+    sn = fma_t(sk, cr, ck * sr);
+    cs = fma_t(ck, cr, -(sk * sr));
+}
+
 // standard normals DIMS of cell `cell` at step `step`, in T
 template <typename T, int DIMS>
 __device__ __forceinline__ void cell_normals(uint64_t seed, uint32_t cell, uint64_t step, T (&eta)[DIMS]) {
@@ -94,7 +118,7 @@ __device__ __forceinline__ void cell_normals(uint64_t seed, uint32_t cell, uint6
         if constexpr(sizeof(T) == 8) {
             const double u1 = ((double)w[2 * h] + 0.5) * 0x1p-32;
             const double u2 = ((double)w[2 * h + 1] + 0.5) * 0x1p-32;
-            const double r = sqrt(-2.0 * log_series_pos(u1));
+            const double r = sqrt_normal(-2.0 * log_series_pos(u1));  // 4.6e-10 .. 46
             double sn, cs;
             sincos_2pi(u2, sn, cs);
             eta[2 * h] = r * cs;
@@ -105,9 +129,9 @@ __device__ __forceinline__ void cell_normals(uint64_t seed, uint32_t cell, uint6
             // logarithm is never positive
             const float u1 = (float)w[2 * h] * 0x1p-32f + 0x1p-33f;
             const float u2 = (float)w[2 * h + 1] * 0x1p-32f + 0x1p-33f;
-            const float r = sqrtf(-2.0f * logf(u1)), th = 6.28318530717958647692f * u2;
+            const float r = sqrtf(-2.0f * logf(u1));
             float sn, cs;
-            sincosf(th, &sn, &cs);
+            sincos_2pi(u2, sn, cs);
             eta[2 * h] = r * cs;
             if(2 * h + 1 < DIMS) eta[2 * h + 1] = r * sn;
         }
@@ -214,8 +238,16 @@ hipError_t launch_noise_cfg(const Params &p, const void *in, void *out, const in
     return hipGetLastError();
 }
 
-// tiles: 1D 256 | 4, 2D 64 x 32 | 4 x 4, 3D 16 x 8 x 8 | 8 x 8 x 8 | 4 x 4 x 4 (the largest N allows;
-// Params::noise_tile selects the earlier 64 x 16 / 8 x 8 x 8 shapes)
+// tiles: 1D 256 | 4, 2D 64 x 32 or 64 x 16 | 4 x 4, 3D 8 x 8 x 8 | 4 x 4 x 4 (the
+// largest N allows; Params::noise_tile picks shape and threads).  The normals
+// bound the step (about 900 of its 1260 issue cycles per wave of cells), so a
+// tile's halo and its share of the chip decide, us per step in FP64:
+//   2D N = 256  64 x 16 / 512 threads 5.3, 64 x 32 / 512 7.1     N = 512  5.7, 7.4
+//      N = 1024 12.9, 11.1    N = 2048 42.9, 40.4
+//   3D N = 32   8 x 8 x 8 / 512 5.9, 16 x 8 x 8 / 512 8.7        N = 64   8.7, 8.9
+//      N = 128  51.0, 60.2 (FP32 32.7, 32.2)
+// Rows of a tile per wave instead of indexed loops: fewer instructions, but no
+// faster (2D N = 1024 13.2): the rounds of rows leave waves idle.
 template <typename T, int DIMS, int MODEL, int MOB>
 hipError_t noise_tiles(const Params &p, const void *in, void *out, const int64_t *step_base, int step_off,
                        hipStream_t s) {
