@@ -59,6 +59,7 @@ struct ch_sys {
     int64_t ckpt_hat_cap = 0;
     int graph_steps = 0;
     int tb = 1;  // time steps per stencil launch (temporal blocking depth)
+    int multi = 0;  // steps per launch of the resident kernels (0: not this size)
     // region shape of the 2D wave kernel's shorter launches (K < tb), which
     // close a step count that tb does not divide: smaller regions give such a
     // launch enough blocks to fill the chip
@@ -394,6 +395,10 @@ extern "C" ch_status ch_sys_create(ch_ctx *ctx, const ch_desc *desc, ch_sys **ou
     if(const char *tb = std::getenv("CH_TB_STEPS")) want = std::atoi(tb);
     s->tb = 1;
     while(s->tb * 2 <= max_k && s->tb * 2 <= want) s->tb *= 2;
+    // grids that one block holds, and 1D: many steps per launch (CH_TB_STEPS pins
+    // the depth of the other kernels instead)
+    if(!is_spectral(desc->integrator) && !noisy && !std::getenv("CH_TB_STEPS"))
+        s->multi = chd::stencil_multi_steps(desc->dims, N);
     if(const char *r = std::getenv("CH_WAVE_CFG")) s->p.wave_cfg = std::max(0, std::min(chd::kWaveCfgs - 1, std::atoi(r)));
     // N >= 1024: 128 x 80 regions for the shorter launches (measured at N = 1024
     // with 8-step launches and a 4-step tail: 0.2635 ms per 100 steps against
@@ -919,6 +924,16 @@ extern "C" ch_status ch_sys_evolve(ch_sys *s, int64_t nsteps) {
     if(s->d.integrator == CH_PSEUDOSPECTRAL) return evolve_spectral(s, nsteps);
     if(s->d.integrator == CH_PSEUDOSPECTRAL_MOBILITY) return evolve_psm(s, nsteps);
     if(has_noise(s)) return evolve_noise(s, nsteps);
+    if(s->multi > 0) {
+        while(nsteps > 0) {
+            const int k = (int)std::min<int64_t>(s->multi, nsteps);
+            HIPCHK(c, chd::stencil_multi(s->p, s->d.precision, s->d.integrator, s->d.model, s->d.mobility, k,
+                                         s->psi[s->cur], s->psi[s->cur ^ 1], c->stream));
+            s->cur ^= 1;
+            nsteps -= k;
+        }
+        return CH_OK;
+    }
     const int G = s->graph_steps;
     // up to 4 G steps, a recurring count is one cached graph of all its launches
     // (below); longer runs replay the G-step graph, then the remainder
@@ -987,7 +1002,7 @@ extern "C" ch_status ch_sys_evolve(ch_sys *s, int64_t nsteps) {
     return CH_OK;
 }
 
-extern "C" int32_t ch_sys_steps_per_launch(const ch_sys *s) { return s ? s->tb : 0; }
+extern "C" int32_t ch_sys_steps_per_launch(const ch_sys *s) { return s ? (s->multi > 0 ? s->multi : s->tb) : 0; }
 
 extern "C" int32_t ch_sys_region_shape(const ch_sys *s) {
     if(!s || s->d.dims != 2 || s->d.N < 64 || is_spectral(s->d.integrator) || is_species(s) || has_noise(s)) return -1;
@@ -1052,7 +1067,7 @@ extern "C" ch_status ch_sys_evolve_observe(ch_sys *s, int64_t nsteps) {
     ch_ctx *c = s->ctx;
     if(s->obs_count == CH_OBS_QUEUE)
         return fail(c, CH_EINVAL, "%d observables already queued: fetch before queueing more", CH_OBS_QUEUE);
-    const bool fusable = !is_species(s) && !is_spectral(s->d.integrator) && !has_noise(s) && s->graph_steps > 0 &&
+    const bool fusable = !is_species(s) && !is_spectral(s->d.integrator) && !has_noise(s) && s->multi == 0 && s->graph_steps > 0 &&
                          nsteps >= s->tb && nsteps <= 4 * (int64_t)s->graph_steps;
     const int par = s->cur;
     if(!fusable || (!(s->oexec[par] && s->osteps[par] == nsteps) && s->oseen[par] != nsteps)) {

@@ -33,6 +33,11 @@ bool adjoint_split3d_ok(const Params &p, int mob);
 int adjoint_split3d_blocks(const Params &p);
 hipError_t adjoint_split3d(const Params &p, int precision, int model, int mob, const void *lam_in, void *lam_out,
                            const void *psi, void *const work[4], bool have_mu, double *gacc, hipStream_t s);
+// many steps per launch on small grids and in 1D (stencil_resident.hip): the most
+// steps one launch advances (0: not this size), and 1 .. that many steps
+int stencil_multi_steps(int dims, int N);
+hipError_t stencil_multi(const Params &p, int precision, int integrator, int model, int mob, int steps, const void *in,
+                         void *out, hipStream_t s);
 // the 3D step in one launch marching along z (Params::tile3d >= 4, N >= 32), and
 // whether it is the faster form
 inline bool march3d_ok(const Params &p) { return p.tile3d >= 4 && p.N >= 32; }

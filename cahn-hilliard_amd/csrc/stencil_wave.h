@@ -105,6 +105,7 @@ __device__ __forceinline__ void row_neighbours(const T (&v)[C][RPW], int j, cons
 //               starts its increment sum from the stored part, and the store
 //               keeps the rounding remainder of psi in it, so the field holds
 //               about 32 significant bits and no rounding accumulates
+// steps (WHOLE, no tape): the number of steps instead of K; no halo limits it.
 // XW (x-whole): the region spans the whole periodic x axis (N == 64 C, gx0 =
 // 0): x neighbours use DPP wave rotates and carry no halo, y keeps its 2K halo.
 enum { UPD_PLAIN = 0, UPD_LAUNCH = 1, UPD_STORED = 2, UPD_LOW8 = 3 };
@@ -112,7 +113,8 @@ template <typename T, int MODEL, int MOB, bool EM, int K, class CFG, bool WHOLE,
           bool XW = false>
 __device__ __forceinline__ void wave_region(const T *__restrict__ in, T *__restrict__ out, const Params &p, int gx0,
                                             int gy0, WaveExchange<T, exchange_fields<MOB, EM>(), CFG::NW, CFG::C> &ex,
-                                            const void *__restrict__ cin = nullptr, void *__restrict__ cout = nullptr) {
+                                            const void *__restrict__ cin = nullptr, void *__restrict__ cout = nullptr,
+                                            int steps = K) {
     static_assert(UPD == UPD_PLAIN || (!EM && !TAPE), "compensated updates for the Euler integrator only");
     static_assert(UPD != UPD_LOW8 || sizeof(T) == 4, "8-bit low-order parts of FP32 fields only");
     static_assert(!(XW && WHOLE), "x-whole regions keep a y halo");
@@ -187,7 +189,7 @@ __device__ __forceinline__ void wave_region(const T *__restrict__ in, T *__restr
 
     const T Mc = (T)p.M;
 #pragma unroll 1
-    for(int s = 0; s < K; s++) {
+    for(int s = 0; s < (WHOLE && !TAPE ? steps : K); s++) {
         // ---- phase 1: mu (and M) from psi
         if constexpr(ACC) {
             // psi of this step from the launch's start value and increments

@@ -170,7 +170,8 @@ ch_status ch_sys_download_mobility(ch_sys *sys, double *mob_host);
 ch_status ch_sys_evolve(ch_sys *sys, int64_t nsteps);
 
 /* Time steps one stencil launch advances (temporal blocking depth; 1 for
- * the pseudospectral integrator).  No reference counterpart: introspection for
+ * the pseudospectral integrator; the most of one launch, 32 to thousands, on 1D
+ * grids and on those that one workgroup holds: 2D N <= 64, 3D N <= 16).  No reference counterpart: introspection for
  * measurement (the reference always does one step per launch,
  * EulerCUDA.cu:60-69).  Override with the CH_TB_STEPS environment variable. */
 int32_t ch_sys_steps_per_launch(const ch_sys *sys);
