@@ -66,12 +66,17 @@ template <int MOB>
 __device__ __forceinline__ MobDeriv<MOB> mob_deriv(const Params &p, double r) {
     MobDeriv<MOB> m{1.0, 0.0, 0.0};
     if constexpr(MOB == CH_MOB_FREE_ENERGY) {
-        const double c = 0.5 * p.tvd, X = wertheim_X(p, r), v = p.valence;
-        const double den = 2.0 * c * r * X + 1.0;
-        const double Xv1 = pow(X, v - 1.0);
+        // one reciprocal for both derivatives, products for the power
+        const double c = 0.5 * p.tvd, v = p.valence;
+        double X = wertheim_X_pos(p, r), q = recip_newton(2.0 * c * r * X + 1.0);
+        if(__builtin_expect(!(r > 0.), 0)) {
+            X = wertheim_X(p, r);
+            q = 1.0 / (2.0 * c * r * X + 1.0);
+        }
+        const double Xv1 = pow_uniform(X, p.valence - 1);
         m.hat = r * Xv1 * X;
-        m.drho = p.M * (Xv1 * X + r * v * Xv1 * (-c * X * X / den));
-        m.ddelta = p.M * r * v * Xv1 * (-v * r * X * X / den);
+        m.drho = p.M * (Xv1 * X + r * v * Xv1 * (-c * X * X * q));
+        m.ddelta = p.M * r * v * Xv1 * (-v * r * X * X * q);
     }
     else if constexpr(MOB == CH_MOB_REGULARISED) {
         const double q = 1.0 / (r + p.rho_min);

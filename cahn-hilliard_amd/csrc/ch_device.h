@@ -71,8 +71,7 @@ __device__ __forceinline__ double fma_const(double a, double b, double c) {
 // exact, s comes from a reciprocal refined by Newton steps and one residual
 // correction, and ln 2 is split into a 31-bit head (e ln2_head exact for any
 // exponent) plus the rest of its value.  Within 2 ulp (worst near m = 1) in
-// some 30 instructions, where the library log spends about 100; zero,
-// negative, infinite and NaN arguments go to log().
+// some 30 instructions, where the library log spends about 100.
 __device__ __forceinline__ double log_series_pos(double x) {  // 0 < x < inf
     double m = __builtin_amdgcn_frexp_mant(x);  // [0.5, 1), denormals included
     int e = __builtin_amdgcn_frexp_exp(x);
@@ -104,9 +103,26 @@ __device__ __forceinline__ double log_series_pos(double x) {  // 0 < x < inf
     return __builtin_fma(ed, ln2_head, __builtin_fma(ed, ln2_rest, lm));
 }
 
+// ln x where x is not in (0, inf): -inf at 0, inf at inf, NaN otherwise.  The
+// library's log (and the mobility's pow) in such a branch would be inlined whole,
+// with its registers: 128 and 46 spilled, for 66 to 116 without, in the 2D
+// free-energy mobility kernels (N = 256 on 64 x 64 regions 9.8 -> 4.8 us per step;
+// euler 4.3 -> 3.35 where densities reach the branch)
+__device__ __forceinline__ double log_outside(double x) {
+    return x == 0. ? -__builtin_inf() : (x > 0. ? x : __builtin_nan(""));
+}
+
 __device__ __forceinline__ double log_series(double x) {
-    if(!(x > 0.0) || x == __builtin_inf()) return log(x);
+    if(__builtin_expect(!(x > 0. && x < __builtin_inf()), 0)) return log_outside(x);
     return log_series_pos(x);
+}
+
+// x^n, n >= 0 the same for all threads
+__device__ __forceinline__ double pow_uniform(double x, int n) {
+#pragma clang fp contract(off)
+    double r = n > 0 ? x : 1.;
+    for(int i = 1; i < n; i++) r *= x;
+    return r;
 }
 
 __device__ __forceinline__ double wertheim_X(const Params &p, double r) {
@@ -170,7 +186,7 @@ __device__ __forceinline__ T fprime(const Params &p, T r) {
                 if(rd > 0.) d += p.valence * log_series_pos(X);
             }
             else {
-                d += log(rd > 0. ? xv : rd);
+                d += log_outside(rd > 0. ? xv : rd);
             }
         }
         return (T)d;
@@ -225,16 +241,10 @@ __device__ __forceinline__ T mobility(const Params &p, T r) {
     }
     else if constexpr(MOB == CH_MOB_FREE_ENERGY) {
         double rd = (double)r;
-        if(rd > 0.) {
-            // X^valence by products: 4 to 10 operations for pow's 200
-            const double X = wertheim_X_pos(p, rd);
-            double Xv = X;
-            for(int i = 1; i < p.valence; i++) Xv *= X;
-            return (T)(rd * (p.M * Xv));
-        }
-        double X = wertheim_X(p, rd);
-        double D = p.M * pow(X, (double)p.valence);
-        return (T)(rd * D);
+        // X^valence by products: 4 to 10 operations for pow's 200
+        double X = wertheim_X_pos(p, rd);
+        if(__builtin_expect(!(rd > 0.), 0)) X = wertheim_X(p, rd);
+        return (T)(rd * (p.M * (X * pow_uniform(X, p.valence - 1))));
     }
     else if constexpr(MOB == CH_MOB_REGULARISED) {
         return (T)p.M * r / (r + (T)p.rho_min);
