@@ -406,6 +406,7 @@ static hipError_t adj_wave(const Params &p, int KA, const void *li, void *lo, co
     case 0: return adj_wave_cfg<T, MODEL, WaveCfg0>(p, KA, li, lo, tape, s_top, gacc, s);
     case 3: return adj_wave_cfg<T, MODEL, WaveCfg3>(p, KA, li, lo, tape, s_top, gacc, s);
     case 5: return adj_wave_cfg<T, MODEL, WaveCfg5>(p, KA, li, lo, tape, s_top, gacc, s);
+    case 9: return adj_wave_cfg<T, MODEL, WaveCfg9>(p, KA, li, lo, tape, s_top, gacc, s);
     default: return adj_wave_cfg<T, MODEL, WaveCfg4>(p, KA, li, lo, tape, s_top, gacc, s);
     }
 }
@@ -449,6 +450,7 @@ int adjoint_tiles(const Params &p, bool em) {
             case 0: t = wave_adj_tiles<WaveCfg0>(N, k); break;
             case 3: t = wave_adj_tiles<WaveCfg3>(N, k); break;
             case 5: t = wave_adj_tiles<WaveCfg5>(N, k); break;
+            case 9: t = wave_adj_tiles<WaveCfg9>(N, k); break;
             default: t = wave_adj_tiles<WaveCfg4>(N, k); break;
             }
             m = std::max(m, t);
@@ -538,6 +540,7 @@ static hipError_t tape_tiles(const Params &p, int K, const void *in, void *out, 
     if constexpr(DIMS == 2) {
         if(N >= 64) {
             if(adj_default_cfg(N) == 5) return tape_wave<T, MODEL, MOB, EM, WaveCfg5>(p, K, in, out, s);
+            if(adj_default_cfg(N) == 9) return tape_wave<T, MODEL, MOB, EM, WaveCfg9>(p, K, in, out, s);
             return tape_wave<T, MODEL, MOB, EM, WaveCfg4>(p, K, in, out, s);
         }
     }

@@ -19,9 +19,11 @@
 
 #include "ch_internal.h"
 
-// default temporal-blocking depth (time steps per stencil launch); the 2D wave
-// kernel's region shape defaults to chd::wave_default_cfg(N)
-static constexpr int kDefaultTB = 8;
+// default region shape and temporal-blocking depth (time steps per stencil launch)
+static chd::WaveRule wave_rule(const ch_desc *d) {
+    return chd::wave_default(d->N, d->model == CH_SIMPLE_WERTHEIM,
+                             d->integrator == CH_EULER_MOBILITY && d->mobility != CH_MOB_CONSTANT);
+}
 
 struct ch_ctx {
     int device = 0;
@@ -259,7 +261,7 @@ static chd::Params make_params(const ch_desc *d) {
         p.k_unit = q;
     p.dcf = d->density_conversion > 0.0 ? d->density_conversion : 1.0;
     }
-    p.wave_cfg = chd::wave_default_cfg(d->N);
+    p.wave_cfg = wave_rule(d).cfg;
     p.adj_cfg = chd::adj_default_cfg(d->N);
     // 3D steps below N = 32: LDS tiles of 16x8x8 with 512 threads, or for
     // SimpleWertheim the two-launch step, which evaluates each cell's FP64 f'
@@ -386,12 +388,12 @@ extern "C" ch_status ch_sys_create(ch_ctx *ctx, const ch_desc *desc, ch_sys **ou
     s->elt = desc->precision == CH_FP64 ? 8 : 4;
     const int N = desc->N;
     s->hat = s->bins / N * (N / 2 + 1);
-    // temporal blocking depth: kDefaultTB, or CH_TB_STEPS (environment) when
+    // temporal blocking depth: wave_rule's, or CH_TB_STEPS (environment) when
     // set, rounded down to a depth the shape has (1 for the pseudospectral path)
     // (1 with noise: one launch per step)
     const bool noisy = desc->integrator == CH_EULER_MOBILITY && desc->with_noise;
     const int max_k = (is_spectral(desc->integrator) || noisy) ? 1 : chd::stencil_max_k(desc->dims, desc->N);
-    int want = kDefaultTB;
+    int want = wave_rule(desc).steps;
     if(const char *tb = std::getenv("CH_TB_STEPS")) want = std::atoi(tb);
     s->tb = 1;
     while(s->tb * 2 <= max_k && s->tb * 2 <= want) s->tb *= 2;
@@ -400,10 +402,10 @@ extern "C" ch_status ch_sys_create(ch_ctx *ctx, const ch_desc *desc, ch_sys **ou
     if(!is_spectral(desc->integrator) && !noisy && !std::getenv("CH_TB_STEPS"))
         s->multi = chd::stencil_multi_steps(desc->dims, N);
     if(const char *r = std::getenv("CH_WAVE_CFG")) s->p.wave_cfg = std::max(0, std::min(chd::kWaveCfgs - 1, std::atoi(r)));
-    // N >= 1024: 128 x 80 regions for the shorter launches (measured at N = 1024
+    // N >= 1024: 128 x 80 regions for the launches shorter than 8 steps (measured at N = 1024
     // with 8-step launches and a 4-step tail: 0.2635 ms per 100 steps against
     // 0.2674 with the 192 x 64 regions of the full launches)
-    s->tail_cfg = N >= 1024 ? 7 : s->p.wave_cfg;
+    s->tail_cfg = N >= 1024 && s->tb == 8 ? 7 : s->p.wave_cfg;
     if(const char *r = std::getenv("CH_WAVE_CFG_TAIL")) s->tail_cfg = std::max(0, std::min(chd::kWaveCfgs - 1, std::atoi(r)));
     if(const char *r = std::getenv("CH_TILE3D")) s->p.tile3d = std::max(0, std::min(5, std::atoi(r)));
     if(const char *r = std::getenv("CH_ADJ_TILE3D")) s->p.adj_tile3d = std::max(0, std::min(2, std::atoi(r)));
@@ -411,7 +413,7 @@ extern "C" ch_status ch_sys_create(ch_ctx *ctx, const ch_desc *desc, ch_sys **ou
     if(const char *r = std::getenv("CH_PSM_FUSE")) s->psm_fuse = std::atoi(r) != 0;
     if(const char *r = std::getenv("CH_ADJ_CFG")) {
         const int v = std::atoi(r);
-        if(v == 0 || v == 3 || v == 4 || v == 5) s->p.adj_cfg = v;
+        if(v == 0 || v == 3 || v == 4 || v == 5 || (v == 9 && N >= 128)) s->p.adj_cfg = v;
     }
     // graph chunk: a multiple of 2 tb launches' worth of steps (parity restored)
     const char *g = std::getenv("CH_GRAPH_STEPS");

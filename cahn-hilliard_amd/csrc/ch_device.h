@@ -18,7 +18,7 @@ struct Params {
     int valence;
     int use_dealias;
     int wave_cfg;          // region shape of the 2D wave kernel (0 .. kWaveCfgs - 1)
-    int adj_cfg;           // region shape of the 2D wave adjoint (0, 3, 4 or 5)
+    int adj_cfg;           // region shape of the 2D wave adjoint (0, 3, 4, 5 or 9)
     int tile3d;            // 3D forward step: LDS tile 0: 16x8x8 / 256 threads, 1: the same / 512, 2: 16x16x4 / 512; 3: two launches (stencil_split.hip); 4, 5: one launch marching along z (stencil_march.hip; 5: the reverse step in two launches)
     int adj_tile3d;        // 3D tile of the euler_mobility adjoint (0: 16x4x4 / 256, 1 (default): 16x8x4 / 512, 2: 16x8x8 / 512)
     int noise_tile;        // tile of the noise step (0: 2D 64x16, 3D 8x8x8 / 256 threads; 1 (default): the same / 512; 2 (default for 2D N >= 1024): 2D 64x32, 3D 16x8x8 / 512)
@@ -416,15 +416,40 @@ __device__ __forceinline__ void mode_q2(const Params &p, int ix, int iy, int iz,
 }
 
 // number of 2D wave-kernel region shapes selectable through Params::wave_cfg
-constexpr int kWaveCfgs = 9;
-// default forward shape, measured on MI355X over shapes 0-8 at 8 steps per
-// launch (FP64 and FP32): 64 x 64 regions of 16 waves up to N = 512, where more,
-// smaller blocks fill the CUs; 192 x 64 at N = 1024 (224 blocks, one per CU);
-// 128 x 80 from N = 2048
-__host__ __device__ constexpr int wave_default_cfg(int N) { return N <= 512 ? 4 : (N == 1024 ? 8 : 7); }
-// reverse sweep and its forward recompute (shapes 0, 3, 4, 5): 128 x 64 regions
-// from N = 512, 64 x 64 below
-__host__ __device__ constexpr int adj_default_cfg(int N) { return N >= 512 ? 5 : 4; }
+constexpr int kWaveCfgs = 10;
+// Default region shape and steps per launch of the forward.  A launch of K steps
+// computes a halo of 2 K cells around each region's interior: deep launches
+// save launches and memory passes, shallow ones save arithmetic, so the depth
+// falls with the work per cell and with the size, where launches weigh less;
+// the regions keep about one block per CU.  us per step in FP64 on MI355X, chosen
+// against shape / steps 4/8 up to N = 512, 8/8 at 1024, 7/8 above:
+//   N                        128         256         512         1024        2048        4096
+//   Landau euler             9/8         9/8         4/8         8/8         7/8         7/4
+//                            0.87, 1.12  0.89, 1.11  1.44        2.51        6.70        21.3, 23.6
+//   Landau, mobility(psi)    9/8         9/8         4/8         8/8         4/2         4/2
+//     (regularised)          1.40, 2.02  1.53, 2.03  2.42        5.00        15.2, 17.6  50.9, 61.0
+//   SimpleWertheim euler     9/8         9/8         9/4         5/4         5/2         5/2
+//                            2.30, 3.07  2.30, 3.07  3.33, 3.58  7.19, 7.98  24.7, 28.8  81.8, 99.4
+//     free-energy mobility   3.45, 4.82  3.45, 4.82  4.83, 5.57  8.98, 10.5  29.3, 38.2  99.8, 130
+struct WaveRule {
+    int cfg, steps;
+};
+__host__ __device__ constexpr WaveRule wave_default(int N, bool wertheim, bool var_mobility) {
+    if(N == 128 || N == 256) return {9, 8};
+    if(N < 512) return {4, 8};
+    if(wertheim) return N == 512 ? WaveRule{9, 4} : (N == 1024 ? WaveRule{5, 4} : WaveRule{5, 2});
+    if(N == 512) return {4, 8};
+    if(N == 1024) return {8, 8};
+    if(var_mobility) return {4, 2};
+    return N == 2048 ? WaveRule{7, 8} : WaveRule{7, 4};
+}
+// reverse sweep and its forward recompute (shapes 0, 3, 4, 5, 9): 128 x 64 regions
+// from N = 512; 64 x 40 at N = 128 and 256, where 64 x 64 leaves three CUs in four
+// idle (record of every 16th state + sweep of 64 steps in FP64, N = 256: 386 -> 356 us,
+// every state kept 282 -> 254); 64 x 64, the whole grid, at 64
+__host__ __device__ constexpr int adj_default_cfg(int N) {
+    return N >= 512 ? 5 : (N >= 128 ? 9 : 4);
+}
 
 // half-spectrum entry q = ((z N) + y) Nh + kx -> (half-axis index ix, iy, iz)
 // as mode_q2 takes them

@@ -175,7 +175,7 @@ ch_status ch_sys_evolve(ch_sys *sys, int64_t nsteps);
  * measurement (the reference always does one step per launch,
  * EulerCUDA.cu:60-69).  Override with the CH_TB_STEPS environment variable. */
 int32_t ch_sys_steps_per_launch(const ch_sys *sys);
-/* Region shape index (0-8) of the 2D register/DPP stencil kernel, -1 for the
+/* Region shape index (0-9) of the 2D register/DPP stencil kernel, -1 for the
  * systems that do not use it (1D, 3D, N < 64, spectral, species, noise).  No
  * reference counterpart: introspection for measurement.  Override with the
  * CH_WAVE_CFG environment variable. */
