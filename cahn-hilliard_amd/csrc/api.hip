@@ -42,6 +42,7 @@ struct ch_sys {
     void *work = nullptr, *rho_hat = nullptr, *twiddles = nullptr;
     void *stage = nullptr;   // bins doubles: host transfers of FP32 fields, mobility
     void *stage2 = nullptr;  // bins elements of T: mobility
+    void *sq_buf = nullptr;  // S(q), shell counts and target of the structure factor
     void *split_mob = nullptr;  // bins elements of T: the cells' mobilities of the two-launch 3D step
     // the 3D euler_mobility reverse step of one cell per thread: nu
     void *adj_split[1] = {nullptr};
@@ -52,6 +53,7 @@ struct ch_sys {
     int64_t ckpt_cap = 0, tape_cap = 0;  // capacities in fields
     int64_t rec_steps = 0, rec_window = 0;
     bool rec_valid = false, rec_full_tape = false;
+    bool rec_last = false;  // the last window's states are on the tape (as recorded)
     hipStream_t aux = nullptr;  // window recompute, overlapped with the adjoint
     hipEvent_t ev_start = nullptr, ev_rec[2] = {nullptr, nullptr}, ev_adj[2] = {nullptr, nullptr};
     // pseudospectral reverse mode: checkpointed spectra, the recompute's spectral
@@ -350,7 +352,7 @@ static void free_sys(ch_sys *s) {
     void *bufs[] = {s->noise_step, s->work, s->rho_hat, s->twiddles, s->stage, s->stage2, s->split_mob, s->partials, s->result,
                     s->ckpt, s->tape, s->lam[0], s->lam[1], s->gacc, s->ckpt_hat, s->ps_rh, s->ps_w,
                     s->ps_spec[0], s->ps_spec[1], s->ps_spec[2], s->ps_real[0], s->ps_real[1],
-                    s->adj_split[0]};
+                    s->adj_split[0], s->sq_buf};
     for(void *b : bufs)
         if(b) (void)hipFree(b);
     for(void *b : s->psm_spec)
@@ -1203,6 +1205,10 @@ static ch_status ensure_spectral(ch_sys *s) {
         const void *src = s->d.precision == CH_FP64 ? (const void *)twd.data() : (const void *)twf.data();
         HIPCHK(c, hipMemcpy(s->twiddles, src, (size_t)N * 2 * s->elt, hipMemcpyHostToDevice));
     }
+    if(!s->sq_buf && hipMalloc(&s->sq_buf, 3 * ch_sq_nshells(N) * sizeof(double)) != hipSuccess) {
+        s->sq_buf = nullptr;
+        return fail(c, CH_ENOMEM, "no device memory for the structure factor");
+    }
     return CH_OK;
 }
 
@@ -1226,15 +1232,13 @@ extern "C" ch_status ch_sys_structure_factor(ch_sys *s, double *Sq, int32_t nshe
     HIPCHK(c, hipSetDevice(c->device));
     ch_status st = ensure_spectral(s);
     if(st != CH_OK) return st;
-    double *buf = nullptr;
-    HIPCHK(c, hipMalloc((void **)&buf, 2 * ns * sizeof(double)));
+    double *buf = (double *)s->sq_buf;
     st = sq_compute(s, ns, buf, buf + ns);
     if(st == CH_OK) {
         hipError_t e = hipMemcpyAsync(Sq, buf, ns * sizeof(double), hipMemcpyDeviceToHost, c->stream);
         if(e == hipSuccess) e = hipStreamSynchronize(c->stream);
         if(e != hipSuccess) st = fail(c, CH_EHIP, "structure factor copy failed: %s", hipGetErrorString(e));
     }
-    (void)hipFree(buf);
     return st;
 }
 
@@ -1248,9 +1252,7 @@ extern "C" ch_status ch_sys_sq_loss(ch_sys *s, const double *target, int32_t nsh
     HIPCHK(c, hipSetDevice(c->device));
     ch_status st = ensure_spectral(s);
     if(st != CH_OK) return st;
-    double *buf = nullptr;
-    HIPCHK(c, hipMalloc((void **)&buf, 3 * ns * sizeof(double)));
-    double *sq = buf, *cnt = buf + ns, *tg = buf + 2 * ns;
+    double *sq = (double *)s->sq_buf, *cnt = sq + ns, *tg = sq + 2 * ns;
     std::vector<double> h(ns);
     hipError_t e = hipMemcpyAsync(tg, target, ns * sizeof(double), hipMemcpyHostToDevice, c->stream);
     if(e == hipSuccess) {
@@ -1266,7 +1268,6 @@ extern "C" ch_status ch_sys_sq_loss(ch_sys *s, const double *target, int32_t nsh
         }
         if(e == hipSuccess) e = hipStreamSynchronize(c->stream);
     }
-    (void)hipFree(buf);
     if(st != CH_OK) return st;
     if(e != hipSuccess) return fail(c, CH_EHIP, "structure-factor loss failed: %s", hipGetErrorString(e));
     if(loss) {
@@ -1742,6 +1743,7 @@ extern "C" ch_status ch_sys_record(ch_sys *s, int64_t nsteps, int32_t ckpt_every
     const bool ps = s->d.integrator == CH_PSEUDOSPECTRAL;
     const size_t hb = (size_t)s->hat * 2 * s->elt;
     s->rec_valid = false;
+    s->rec_last = false;
     s->rec_full_tape = ckpt_every == 0;
     s->rec_window = ckpt_every == 0 ? nsteps : std::min<int64_t>(ckpt_every, nsteps);
     const int64_t nck = (nsteps + s->rec_window - 1) / s->rec_window;
@@ -1790,6 +1792,17 @@ extern "C" ch_status ch_sys_record(ch_sys *s, int64_t nsteps, int32_t ckpt_every
         for(int64_t k = 0; k < nck; k++) {
             HIPCHK(c, hipMemcpyAsync(field_at(s->ckpt, k, fb), s->psi[s->cur], fb, hipMemcpyDeviceToDevice, c->stream));
             const int64_t steps = std::min<int64_t>(s->rec_window, nsteps - k * s->rec_window);
+            if(k == nck - 1) {
+                // the last window straight onto its tape: the sweep starts there, with
+                // nothing to overlap its recompute with
+                const size_t sb = tape_slot(s);
+                char *tape = field_at(s->tape, (k & 1) * s->rec_window, sb);
+                HIPCHK(c, hipMemcpyAsync(tape, s->psi[s->cur], fb, hipMemcpyDeviceToDevice, c->stream));
+                HIPCHK(c, tape_steps(s, tape, 0, steps, c->stream));
+                HIPCHK(c, hipMemcpyAsync(s->psi[s->cur], field_at(tape, steps, sb), fb, hipMemcpyDeviceToDevice, c->stream));
+                s->rec_last = true;
+                break;
+            }
             ch_status st = ch_sys_evolve(s, steps);
             if(st != CH_OK) return st;
         }
@@ -1826,7 +1839,10 @@ static ch_status adjoint_core(ch_sys *s, double *grads) {
         const int64_t start = k * W, len = std::min<int64_t>(W, T - start);
         const int b = (int)(k & 1);
         void *tape = recompute ? field_at(s->tape, b * W, tape_slot(s)) : s->tape;
-        if(recompute) {
+        // the record's own tape of the last window, until a later window takes its buffer
+        const bool recorded = s->rec_last && k == nck - 1;
+        if(k == nck - 3) s->rec_last = false;
+        if(recompute && !recorded) {
             if(used[b]) HIPCHK(c, hipStreamWaitEvent(s->aux, s->ev_adj[b], 0));
             HIPCHK(c, hipMemcpyAsync(tape, field_at(s->ckpt, k, fb), fb, hipMemcpyDeviceToDevice, s->aux));
             if(ps) {
