@@ -1691,10 +1691,17 @@ static bool grow(void **buf, int64_t &cap, int64_t fields, size_t field_bytes) {
 
 static char *field_at(void *base, int64_t i, size_t field_bytes) { return (char *)base + (size_t)i * field_bytes; }
 
-// the 3D euler_mobility reverse sweep in three launches per step
+// the 3D euler_mobility reverse sweep in two launches per step
 // (chd::adjoint_split3d) and its window recompute in two
 static bool adj_split(const ch_sys *s) {
     return s->d.dims == 3 && s->d.integrator == CH_EULER_MOBILITY && chd::adjoint_split3d_ok(s->p, s->d.mobility);
+}
+
+// ... or, with the mobilities and mu on the tape, in one launch each
+// (chd::adj_march3d, chd::march3d_record)
+static bool adj_march(const ch_sys *s) {
+    return adj_split(s) && chd::march3d_ok(s->p) && s->d.model == CH_SIMPLE_WERTHEIM &&
+           chd::march3d_reverse_better(s->p, s->d.precision);
 }
 
 // Tape slots: psi_t, and with the three-launch reverse step also mu_t and the
@@ -1707,6 +1714,8 @@ static hipError_t tape_step1(ch_sys *s, const void *in, void *out, hipStream_t s
     const ch_desc &d = s->d;
     if(adj_split(s)) {
         const size_t fb = s->bins * s->elt;
+        if(adj_march(s))
+            return chd::march3d_record(s->p, d.precision, d.mobility, in, out, (char *)in + fb, (char *)in + 2 * fb, st);
         return chd::stencil_split3d(s->p, d.precision, d.integrator, d.model, d.mobility, in, out, (char *)in + fb,
                                     (char *)in + 2 * fb, st);
     }
@@ -1747,10 +1756,11 @@ extern "C" ch_status ch_sys_record(ch_sys *s, int64_t nsteps, int32_t ckpt_every
     s->rec_full_tape = ckpt_every == 0;
     s->rec_window = ckpt_every == 0 ? nsteps : std::min<int64_t>(ckpt_every, nsteps);
     const int64_t nck = (nsteps + s->rec_window - 1) / s->rec_window;
-    // checkpointed: two window tapes, one recomputed while the other is swept;
-    // the pseudospectral full tape also keeps the final state
-    const int64_t tape_fields = s->rec_full_tape ? nsteps + (ps ? 1 : 0) : 2 * s->rec_window;
-    if(adj_split(s))
+    // checkpointed: two window tapes, one recomputed while the other is swept,
+    // and the state after the last window; the pseudospectral full tape also
+    // keeps the final state
+    const int64_t tape_fields = s->rec_full_tape ? nsteps + (ps ? 1 : 0) : 2 * s->rec_window + (ps ? 0 : 1);
+    if(adj_split(s) && !adj_march(s))
         for(void *&b : s->adj_split)
             if(!b && hipMalloc(&b, fb) != hipSuccess) {
                 b = nullptr;
@@ -1877,6 +1887,13 @@ static ch_status adjoint_core(ch_sys *s, double *grads) {
         if(adj_split(s)) {
             for(int64_t t = len - 1; t >= 0; t--) {
                 char *slot = field_at(tape, t, tape_slot(s));
+                if(adj_march(s)) {
+                    const void *const rec[3] = {slot, slot + fb, slot + 2 * fb};
+                    HIPCHK(c, chd::adj_march3d(s->p, s->d.precision, s->d.mobility, s->lam[li], s->lam[li ^ 1], rec,
+                                               s->gacc, ms));
+                    li ^= 1;
+                    continue;
+                }
                 void *const w[4] = {slot + fb, slot + 2 * fb, s->adj_split[0], nullptr};
                 HIPCHK(c, chd::adjoint_split3d(s->p, s->d.precision, s->d.model, s->d.mobility, s->lam[li],
                                                s->lam[li ^ 1], slot, w, true, s->gacc, ms));
