@@ -1120,7 +1120,7 @@ hipError_t fft2_inverse(const SpectralArgs &a, void *out, hipStream_t s) {
 // two modes of the full spectrum.  One block per shell, four lanes per row: each
 // row's run of modes starts at a bound below the annulus and ends at the first
 // mode above it, in a fixed order (deterministic sums).  Visiting all of the
-// shell's bounding box instead took 53 us at N = 256; now 7.
+// shell's bounding box instead took 53 us at N = 256; now 9.
 __device__ __forceinline__ int sq_shell(int kx, int iy) { return (int)rint(sqrt((double)(kx * kx + iy * iy))); }
 
 template <typename T>

@@ -11,7 +11,7 @@
 // between them take 22 (37): below N = 1024 each launch lasts 4 to 6.5 us
 // whatever it does (a kernel start plus one round trip to lines that another
 // XCD wrote), so the step's time is mostly its number of launches.  2D N = 512
-// FP64 on MI355X: 99 -> 43 us per step.
+// FP64 on MI355X: 99 -> 41 us per step.
 // The per-entry operations and their order are those of the element-wise
 // kernels (psm_ops.h, psm.hip).
 #include <type_traits>
@@ -365,14 +365,26 @@ struct LastAxis {
         stride = DIMS == 2 ? Nh : (long)p.N * Nh;
     }
     __device__ __forceinline__ size_t at(int j) const { return base + (size_t)j * stride; }
+    // entry j of line l in a line-major field
+    __device__ __forceinline__ size_t own(const Params &p, int l, int j) const { return (size_t)l * p.N + j; }
     __device__ __forceinline__ int iy(int j) const { return DIMS == 2 ? j : mid; }
     __device__ __forceinline__ int iz(int j) const { return DIMS == 2 ? 0 : j; }
 };
 
 // f_hat of each line (kept in FH), mu_hat = (f_hat + 2k q^2 rho_hat) deal, and
 // per axis d the inverse transform of (i k_d) deal mu_hat
+// Blocks of one line keep f_hat, which only these two passes touch, line-major
+// (entry j of line l at l N + j), and in 2D rho_hat too from the first step's join
+// to the last one's (lm: rho_hat is line-major).  A line's entries in the half
+// spectrum lie a row apart, one 128 B line of memory each for 16 B of use, and
+// that traffic, not the transforms, bounds both passes (running a line's axes
+// beside each other changed nothing; other row strides neither).  2D on MI355X, us
+// per step, all fields in the half spectrum's layout -> f_hat -> rho_hat too:
+//   N = 256   FP64 31.9 -> 31.2 -> 31.2   FP32 28.6 -> 28.0 -> 28.0
+//   N = 512        44.0 -> 41.5 -> 40.8        36.2 -> 33.2 -> 32.2
+//   N = 1024       89.2 -> 85.8 -> 80.2        62.1 -> 59.3 -> 53.5
 template <typename T, class ENG, int DIMS>
-__global__ __launch_bounds__(ENG::NT) void k_psm_split(const C2<T> *__restrict__ W, const C2<T> *__restrict__ RH,
+__global__ __launch_bounds__(ENG::NT) void k_psm_split(const C2<T> *__restrict__ W, const C2<T> *__restrict__ RH, bool lm,
                                                        C2<T> *__restrict__ FH, Fields<C2<T>> Gs,
                                                        const C2<T> *__restrict__ table, Params p, int lines) {
 #pragma clang fp contract(off)
@@ -390,13 +402,16 @@ __global__ __launch_bounds__(ENG::NT) void k_psm_split(const C2<T> *__restrict__
 #pragma unroll
     for(int i = 0; i < E; i++) v[i] = W[ax.at(eng.in(i))];
 #pragma unroll
-    for(int i = 0; i < E; i++) mu[i] = RH[ax.at(eng.freq(i))];
+    for(int i = 0; i < E; i++) {
+        const int j = eng.freq(i);
+        mu[i] = RH[lm ? ax.own(p, l, j) : ax.at(j)];
+    }
     eng.finish(table);
     eng.forward(v);
 #pragma unroll
     for(int i = 0; i < E; i++) {
         const int j = eng.freq(i);
-        if(on) FH[ax.at(j)] = v[i];
+        if(on) FH[ENG::NL == 1 ? ax.own(p, l, j) : ax.at(j)] = v[i];
         double k2, deal;
         mode_q2(p, ax.ix, ax.iy(j), ax.iz(j), k2, deal);
         if(!p.use_dealias) deal = 1.0;
@@ -421,7 +436,8 @@ __global__ __launch_bounds__(ENG::NT) void k_psm_split(const C2<T> *__restrict__
 // inverse transform of rho_hat / N^d into W
 template <typename T, class ENG, int DIMS>
 __global__ __launch_bounds__(ENG::NT) void k_psm_join(Fields<C2<T>> Gs, const C2<T> *__restrict__ FH,
-                                                      C2<T> *__restrict__ RH, C2<T> *__restrict__ W,
+                                                      const C2<T> *RH, bool lm, C2<T> *RO, bool lm_out,
+                                                      C2<T> *__restrict__ W,
                                                       const C2<T> *__restrict__ table, Params p, int lines,
                                                       const double *__restrict__ parts, int nparts) {
 #pragma clang fp contract(off)
@@ -442,8 +458,9 @@ __global__ __launch_bounds__(ENG::NT) void k_psm_join(Fields<C2<T>> Gs, const C2
         for(int i = 0; i < E; i++) g[a][i] = Gs.f[a][ax.at(eng.in(i))];
 #pragma unroll
     for(int i = 0; i < E; i++) {
-        r[i] = RH[ax.at(eng.freq(i))];
-        f[i] = FH[ax.at(eng.freq(i))];
+        const int j = eng.freq(i);
+        r[i] = RH[lm ? ax.own(p, l, j) : ax.at(j)];
+        f[i] = FH[ENG::NL == 1 ? ax.own(p, l, j) : ax.at(j)];
         dv[i] = T2{0, 0};
     }
     M0Reader rd;
@@ -476,7 +493,8 @@ __global__ __launch_bounds__(ENG::NT) void k_psm_join(Fields<C2<T>> Gs, const C2
 #pragma unroll
     for(int i = 0; i < E; i++)
         if(on) {
-            RH[ax.at(eng.freq(i))] = r[i];
+            const int j = eng.freq(i);
+            RO[lm_out ? ax.own(p, l, j) : ax.at(j)] = r[i];
             W[ax.at(eng.in(i))] = dv[i];
         }
 }
@@ -554,19 +572,24 @@ struct Chain {
         using Eng = Engine<T, LOG2N, DIMS>;
         const Fields<T2> W{{(T2 *)B.a.work, nullptr, nullptr}};
         const int blocks = col_blocks(lines, Eng::NL);
+        constexpr bool keep = DIMS == 2 && Eng::NL == 1;
         int nparts = 0;
         hipError_t e = psm_mobility(B, B.max_parts, nparts, s);
         if(e == hipSuccess) e = spec_x_forward(B.a, B.a.rho, B.a.work, true, s);
         if(e == hipSuccess) nparts = reduce(nparts);
         for(int64_t t = 0; t < nsteps && e == hipSuccess; t++) {
             if((e = y_pass(W, 1, false)) != hipSuccess) return e;
+            const bool lm = keep && t > 0;  // 2D: the third component's spectrum is free
+            const T2 *RH = (const T2 *)(lm ? B.muh : B.a.rho_hat);
             hipLaunchKernelGGL((k_psm_split<T, Eng, DIMS>), dim3(blocks), dim3(Eng::NT), 0, s, W.f[0],
-                               (const T2 *)B.a.rho_hat, (T2 *)B.fh, G, tw, p, lines);
+                               RH, lm, (T2 *)B.fh, G, tw, p, lines);
             if((e = y_pass(G, DIMS, true)) != hipSuccess) return e;
             row<0, CH_LANDAU>(G, DIMS, nparts);
             if((e = y_pass(G, DIMS, false)) != hipSuccess) return e;
-            hipLaunchKernelGGL((k_psm_join<T, Eng, DIMS>), dim3(blocks), dim3(Eng::NT), 0, s, G, (const T2 *)B.fh,
-                               (T2 *)B.a.rho_hat, W.f[0], tw, p, lines, (const double *)B.max_parts, nparts);
+            const bool lmo = keep && t + 1 < nsteps;
+            hipLaunchKernelGGL((k_psm_join<T, Eng, DIMS>), dim3(blocks), dim3(Eng::NT), 0, s, G, (const T2 *)B.fh, RH, lm,
+                               lmo ? (T2 *)B.muh : (T2 *)B.a.rho_hat, lmo, W.f[0], tw, p, lines,
+                               (const double *)B.max_parts, nparts);
             if((e = y_pass(W, 1, true)) != hipSuccess) return e;
             if(t + 1 < nsteps) {
                 if(B.a.model == CH_LANDAU) row<1, CH_LANDAU>(W, 1, 0);
