@@ -1469,7 +1469,7 @@ extern "C" ch_status ch_batch_create_ex(ch_ctx *ctx, int32_t n, const ch_desc *d
     if(!b->tuned && tune_lookup(tune_key(b), b->shape, b->tb)) b->tuned = true;
     bool ok = hipMalloc(&b->buf[0], b->total * b->elt) == hipSuccess && hipMalloc(&b->buf[1], b->total * b->elt) == hipSuccess &&
               hipMalloc((void **)&b->reps, n * sizeof(chd::BatchRep)) == hipSuccess &&
-              hipMalloc(&b->stage, maxbins * 8) == hipSuccess && hipMalloc((void **)&b->result, 2 * n * sizeof(double)) == hipSuccess;
+              hipMalloc(&b->stage, maxbins * 8) == hipSuccess && hipMalloc((void **)&b->result, 2 * (size_t)n * (1 + chd::kBatchObsParts) * sizeof(double)) == hipSuccess;
     if(ok && (compensation == CH_COMP_STORED || compensation == CH_COMP_LOW8)) {
         const size_t bytes = b->total * b->comp_elt();
         ok = hipMalloc(&b->comp[0], bytes) == hipSuccess && hipMalloc(&b->comp[1], bytes) == hipSuccess &&
