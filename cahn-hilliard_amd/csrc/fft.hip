@@ -343,6 +343,55 @@ __global__ __launch_bounds__(64) void k_colw(const typename Complex<T>::type *__
     for(int m = 0; m < E; m++) dst[base + (size_t)(lane + 64 * m) * stride] = v[m];
 }
 
+// ---- the 2D column pass up to N = 512 on the line engines (line_fft.h), whose
+// blocks hold few lines, so that N / 2 + 1 lines reach many CUs; blocks of one line
+// (N = 256, 512) keep rho_hat line-major.  INIT: the forward transform of src into
+// rho_hat; else forward, spectral update and inverse, src -> dst.  2D chain on
+// MI355X, us per step, k_col / k_colw -> this:
+//   FP64  N = 64 13.5 -> 11.0   128 14.3 -> 11.7   256 15.4 -> 12.6   512 15.7 -> 14.5
+//   FP32         12.2 ->  9.9       13.0 -> 10.6       13.6 -> 11.1       13.6 -> 12.0
+template <typename T, class ENG, bool INIT>
+__global__ __launch_bounds__(ENG::NT) void k_cole(const typename Complex<T>::type *src, typename Complex<T>::type *dst,
+                                                  typename Complex<T>::type *rho_hat,
+                                                  const typename Complex<T>::type *__restrict__ table, Params p, int lines) {
+    using T2 = typename Complex<T>::type;
+    constexpr int E = ENG::E, n = ENG::n, Nh = n / 2 + 1;
+    __shared__ typename ENG::Smem sm;
+    const int l0 = xcd_tile(blockIdx.x, gridDim.x) * ENG::NL;
+    if(l0 >= lines) return;  // grid padded to a multiple of 8 blocks
+    ENG eng(sm);
+    eng.begin(table);
+    const bool on = ENG::NL == 1 || l0 + eng.line() < lines;
+    const int l = on ? l0 + eng.line() : l0;
+    auto rh_at = [&](int j) -> size_t { return ENG::NL == 1 ? (size_t)l * n + j : (size_t)j * Nh + l; };
+    T2 v[E], rh[INIT ? 1 : E];
+#pragma unroll
+    for(int i = 0; i < E; i++) v[i] = src[(size_t)eng.in(i) * Nh + l];
+    if constexpr(!INIT) {
+#pragma unroll
+        for(int i = 0; i < E; i++) rh[i] = rho_hat[rh_at(eng.freq(i))];
+    }
+    eng.finish(table);
+    eng.forward(v);
+    if constexpr(INIT) {
+#pragma unroll
+        for(int i = 0; i < E; i++)
+            if(on) rho_hat[rh_at(eng.freq(i))] = v[i];
+    }
+    else {
+        const T inv_bins = (T)p.inv_bins;
+#pragma unroll
+        for(int i = 0; i < E; i++) v[i] = spectral_update<T, T2>(p, l, eng.freq(i), 0, v[i], rh[i], inv_bins);
+        eng.inverse(v);
+#pragma unroll
+        for(int i = 0; i < E; i++)
+            if(on) {
+                rho_hat[rh_at(eng.freq(i))] = rh[i];
+                dst[(size_t)eng.in(i) * Nh + l] = v[i];
+            }
+    }
+}
+
 // ---- two waves per line of n = 2 n2 points (n2 = 64 E): the axis pass for
 // n = 1024 and 2048, where one wave's chain of transform passes, not memory,
 // bounds the single-wave kernel (a 2D N = 1024 grid has only 513 lines).
@@ -763,7 +812,14 @@ static void launch_col(const typename Complex<T>::type *src, typename Complex<T>
                            lines, P, ls, stride, axis, 0, rhl ? 1 : 0);
         return;
     }
-    (void)rhl;
+    if constexpr(LOG2N >= 2 && LOG2N <= 9 && (MODE == 0 || MODE == 2)) {
+        if(rhl) {
+            using Eng = Engine<T, LOG2N, 2>;
+            hipLaunchKernelGGL((k_cole<T, Eng, MODE == 0>), dim3(col_blocks(lines, Eng::NL)), dim3(Eng::NT), 0, s, src, dst,
+                               MODE == 0 ? dst : rh, tw, p, lines);
+            return;
+        }
+    }
     if constexpr(wave_len<LOG2N>()) {
         (void)contig;
         hipLaunchKernelGGL((k_colw<T, MODE, LOG2N>), dim3((lines + 7) / 8 * 8), dim3(64), 0, s, src, dst, rh, tw, p, lines,
@@ -815,7 +871,7 @@ static hipError_t ps_chain_t(const SpectralArgs &a, hipStream_t s, int64_t nstep
     T2 *W = (T2 *)a.work, *RH = (T2 *)a.rho_hat;
     const bool landau = a.model == CH_LANDAU;
     const size_t bins = (size_t)rows * N;
-    const bool rhl = a.rh_lines && dims == 2 && (LOG2N == 10 || LOG2N == 11);
+    const bool rhl = a.rh_lines && dims == 2 && LOG2N <= 11;
     const bool planes = dims == 3 && plane_len<T>(LOG2N);
     if constexpr(plane_len<T>(LOG2N)) {
         if(planes && init) {

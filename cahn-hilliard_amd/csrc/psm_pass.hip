@@ -14,8 +14,6 @@
 // FP64 on MI355X: 99 -> 41 us per step.
 // The per-entry operations and their order are those of the element-wise
 // kernels (psm_ops.h, psm.hip).
-#include <type_traits>
-
 #include "line_fft.h"
 #include "psm_ops.h"
 
@@ -245,112 +243,6 @@ __global__ __launch_bounds__(64 * NR) void k_psm_roww(Fields<C2<T>> Ws, const C2
     if(KIND == 1 && lane == 0) parts[row] = mx;
 }
 
-// ------------------------------------------------------------------ line engines
-// A block's transform of its lines, entries in registers: entry i of a thread
-// is entry in(i) of its line before a forward and after an inverse transform,
-// and entry freq(i) after a forward and before an inverse one.  begin() issues
-// the loads of the twiddles, finish() (after the line's loads) stages them.
-
-// NLC lines per block in LDS (LineFFT); thread t works on line t % NLC
-template <typename T2, int LOG2N, int NLC>
-struct LdsEngine {
-    using G = FftGeom<LOG2N, NLC>;
-    static constexpr int E = 4, NT = G::NT, NL = NLC, n = G::n;
-    struct Smem { T2 buf[padded(G::E)]; };
-    LineFFT<T2, LOG2N, NLC> fft;
-    T2 *buf;
-    int lb, j0;
-    __device__ __forceinline__ LdsEngine(Smem &sm) : buf(sm.buf), lb(threadIdx.x % NLC), j0(threadIdx.x / NLC) {}
-    __device__ __forceinline__ void begin(const T2 *table) { fft.prefetch(table, 1); }
-    __device__ __forceinline__ void finish(const T2 *) {}
-    __device__ __forceinline__ int line() const { return lb; }
-    __device__ __forceinline__ int in(int i) const { return j0 + i * (NT / NLC); }
-    __device__ __forceinline__ int freq(int i) const { return in(i); }
-    template <bool INV>
-    __device__ __forceinline__ void run(T2 (&v)[E]) {
-        __syncthreads();  // the previous transform's reads
-#pragma unroll
-        for(int i = 0; i < E; i++) buf[pidx(lb * n + in(i))] = v[i];
-        __syncthreads();
-        fft.template run<INV>(buf);
-#pragma unroll
-        for(int i = 0; i < E; i++) v[i] = buf[pidx(lb * n + in(i))];
-    }
-    __device__ __forceinline__ void forward(T2 (&v)[E]) { run<false>(v); }
-    __device__ __forceinline__ void inverse(T2 (&v)[E]) { run<true>(v); }
-};
-
-// two waves per line (the scheme of k_colw2): half-length transforms of the
-// even and odd entries joined by one exchange.  N = 512 uses the 256-point
-// four-pass transform, so that its 257 lines fill 514 waves.
-template <typename T2, int LOG2N>
-struct TwoWaveEngine {
-    static constexpr int n = 1 << LOG2N, n2 = n / 2, E = n2 / 64, NT = 128, NL = 1;
-    using F = std::conditional_t<LOG2N == 9, WaveFFT4<T2>, WaveFFT<T2, LOG2N == 9 ? 9 : LOG2N - 1>>;
-    using Stage = TwiddleStage<T2, n>;
-    static constexpr int TWR = Stage::on ? n / NT : 1;
-    struct Smem {
-        T2 lds[2][F::LDS];
-        Stage stage;
-    };
-    Smem &sm;
-    const T2 *tw = nullptr;
-    T2 *own, *other;
-    int lane, h;
-    T2 twr[TWR];
-    __device__ __forceinline__ TwoWaveEngine(Smem &s) : sm(s) {
-        lane = threadIdx.x & 63;
-        h = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        own = sm.lds[h];
-        other = sm.lds[h ^ 1];
-    }
-    __device__ __forceinline__ void begin(const T2 *table) { sm.stage.template load<NT>(table, threadIdx.x, twr); }
-    __device__ __forceinline__ void finish(const T2 *table) {
-        tw = sm.stage.template store<NT>(table, threadIdx.x, twr);  // visible after the next barrier
-    }
-    __device__ __forceinline__ int line() const { return 0; }
-    __device__ __forceinline__ int in(int m) const { return 2 * (lane + 64 * m) + h; }
-    __device__ __forceinline__ int freq(int m) const { return lane + 64 * m + h * n2; }
-    template <bool INV>
-    __device__ __forceinline__ void half(T2 (&v)[E]) {
-        if constexpr(LOG2N == 9) {
-            lds_barrier();
-            F::template run<INV>(lane, v, own, tw, 2);
-        }
-        else {
-            wave_transform<T2, LOG2N - 1, INV>(lane, v, own, tw, 2);
-        }
-    }
-    __device__ __forceinline__ void forward(T2 (&v)[E]) {
-        half<false>(v);
-#pragma unroll
-        for(int m = 0; m < E; m++)
-            if(h == 1) v[m] = cmul(v[m], tw[lane + 64 * m]);
-        wave_lds_sync();  // the other wave has not read this buffer since the transform's barrier
-#pragma unroll
-        for(int m = 0; m < E; m++) own[lane + 64 * m] = v[m];
-        lds_barrier();
-#pragma unroll
-        for(int m = 0; m < E; m++) {
-            const T2 o = other[lane + 64 * m];
-            v[m] = h == 0 ? cadd(v[m], o) : csub(o, v[m]);
-        }
-    }
-    __device__ __forceinline__ void inverse(T2 (&v)[E]) {
-        lds_barrier();
-#pragma unroll
-        for(int m = 0; m < E; m++) own[lane + 64 * m] = v[m];
-        lds_barrier();
-#pragma unroll
-        for(int m = 0; m < E; m++) {
-            const T2 o = other[lane + 64 * m];
-            if(h == 0) v[m] = cadd(v[m], o);
-            else v[m] = cmul(csub(o, v[m]), conj_(tw[lane + 64 * m]));
-        }
-        half<true>(v);
-    }
-};
-
 // the lines of the last axis: line l, entry j at base + j stride, and its modes
 template <int DIMS>
 struct LastAxis {
@@ -500,17 +392,6 @@ __global__ __launch_bounds__(ENG::NT) void k_psm_join(Fields<C2<T>> Gs, const C2
 }
 
 // ------------------------------------------------------------------ host side
-// lines per block of the LDS engine: in 2D few (N / 2 + 1 lines have to reach
-// many CUs, 64 threads per block), in 3D as the axis passes (k_col)
-template <int LOG2N, int DIMS>
-constexpr int engine_lines() {
-    return DIMS == 3 ? ColLines<LOG2N>::value : (LOG2N >= 8 ? 1 : (256 >> LOG2N));
-}
-
-template <typename T, int LOG2N, int DIMS>
-using Engine = std::conditional_t<(LOG2N >= 9 && LOG2N <= 11), TwoWaveEngine<C2<T>, (LOG2N >= 9 && LOG2N <= 11) ? LOG2N : 10>,
-                                  LdsEngine<C2<T>, LOG2N, engine_lines<LOG2N, DIMS>()>>;
-
 template <typename T, int LOG2N, int DIMS>
 struct Chain {
     using T2 = C2<T>;
