@@ -49,9 +49,14 @@ struct FftGeom {
     static constexpr int NP4 = LOG2N / 2;  // radix-4 passes
 };
 
-// lines of n <= 256 are packed four-per-1024 elements (NT = 256)
+// Rows per block of the LDS row passes: as many as one wave takes (NT = 64), so that
+// the few rows of a 2D grid reach many CUs (256-thread blocks left N = 256 on 32 of
+// them); n <= 4 as 256 threads take.  2D on MI355X, us per step, 256 threads -> 64:
+// pseudospectral FP64 N = 64 11.1 -> 9.9, 128 11.8 -> 10.4, 256 12.7 -> 11.2 (FP32 10.4
+// -> 9.2, 10.7 -> 9.6, 11.2 -> 10.1); splitting step FP64 27.4 -> 25.2, 29.3 -> 26.3,
+// 31.3 -> 28.0; 3D N = 32 to 128 equal.
 template <int LOG2N>
-struct PackedLines { static constexpr int value = LOG2N >= 8 ? 1 : (1 << (10 - LOG2N)); };
+struct PackedLines { static constexpr int value = LOG2N >= 8 ? 1 : (1 << ((LOG2N <= 2 ? 10 : 8) - LOG2N)); };
 
 template <typename T2, int LOG2N, int NLINES>
 struct LineFFT {

@@ -90,12 +90,12 @@ struct Fields {
 // (W = its half spectrum, mob read, M0 from parts).  KIND 1: between two steps
 // (mob written, parts[block] = the block's largest mobility; the densities
 // instead under the free-energy rule).
-template <typename T, int KIND, int MODEL, int LOG2N>
-__global__ __launch_bounds__((FftGeom<LOG2N, PackedLines<LOG2N>::value>::NT)) void k_psm_row(
+template <typename T, int KIND, int MODEL, int LOG2N, int NLR>
+__global__ __launch_bounds__((FftGeom<LOG2N, NLR>::NT)) void k_psm_row(
     Fields<C2<T>> Ws, const C2<T> *__restrict__ tw, Params p, int rows, long rs, T *__restrict__ mob, int rule,
     double *__restrict__ parts, int nparts) {
     using T2 = C2<T>;
-    using G = FftGeom<LOG2N, PackedLines<LOG2N>::value>;
+    using G = FftGeom<LOG2N, NLR>;
     constexpr int n = G::n, N = 2 * n, nl = G::NL, NT = G::NT, Nh = n + 1;
     __shared__ T2 buf[padded(G::E + nl)];
     T2 *__restrict__ W = Ws.f[blockIdx.y];
@@ -411,8 +411,11 @@ struct Chain {
     }
     static int row_parts(int rows) {
         if constexpr(wave_len<LX>()) return rows;
-        else return (rows + PackedLines<LX>::value - 1) / PackedLines<LX>::value;
+        else return (rows + row_lines() - 1) / row_lines();
     }
+    // rows per block of k_psm_row; 3D from N = 128 four times as many, which keeps its
+    // partial maxima within kMaxParts (N = 128: no reduction launch of their own)
+    static constexpr int row_lines() { return DIMS == 3 && LX >= 6 && LX < 8 ? 1 << (10 - LX) : PackedLines<LX>::value; }
     template <int KIND, int MODEL>
     void row(Fields<T2> W, int nf, int nparts) {
         T *field = (T *)(KIND == 1 && B.mob_rule == CH_MOB_FREE_ENERGY ? B.a.rho : B.mob);
@@ -429,8 +432,8 @@ struct Chain {
             else go(std::integral_constant<int, CH_MOB_FREE_ENERGY>{});
         }
         else {
-            constexpr int NL = PackedLines<LX>::value;
-            hipLaunchKernelGGL((k_psm_row<T, KIND, MODEL, LX>), dim3((rows + NL - 1) / NL, nf),
+            constexpr int NL = row_lines();
+            hipLaunchKernelGGL((k_psm_row<T, KIND, MODEL, LX, NL>), dim3((rows + NL - 1) / NL, nf),
                                dim3(FftGeom<LX, NL>::NT), 0, s, W, tw, p, rows, Nh, field, B.mob_rule, B.max_parts,
                                nparts);
         }
