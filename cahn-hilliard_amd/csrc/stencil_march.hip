@@ -18,10 +18,10 @@
 //                                   N = 32     N = 64     N = 128      N = 256
 //   Landau euler        FP32   2.8 / 4.8  3.5 / 4.6  8.2 / 13.1  41.8 / 82.4
 //                       FP64   3.1 / 5.4  4.0 / 5.3 11.5 / 17.5  62.9 / 118
-//   Wertheim, linear M  FP64   4.4 / 7.2  6.3 / 8.2 20.6 / 27.7   145 / 284
-//            constant M FP64   4.2 / 5.9  5.9 / 6.8 17.9 / 20.4   119 / 188
+//   Wertheim, linear M  FP64   4.7 / 7.4  6.6 / 8.5 21.8 / 28.1   126 / 282
+//            constant M FP64   4.4 / 6.1  6.1 / 7.0 19.0 / 20.9   107 / 179
 //                       FP32   4.0 / 4.8  5.3 / 5.1 14.9 / 13.5   103 / 90
-//            free-energy M FP64 4.9 / 7.1 6.8 / 7.1 21.3 / 30.5   153 / 248
+//            free-energy M FP64 4.9 / 7.3 6.9 / 7.3 22.3 / 31.9   128 / 215
 // FP32 SimpleWertheim with constant mobility moves half the bytes for the same
 // FP64 f', so there the launch that evaluates f' once per cell stays ahead from
 // N = 64 (march3d_better).  Chunks of 8 planes from N = 128 (16: 8.9 us for
