@@ -1722,17 +1722,17 @@ static bool adj_split(const ch_sys *s) {
     return s->d.dims == 3 && s->d.integrator == CH_EULER_MOBILITY && chd::adjoint_split3d_ok(s->p, s->d.mobility);
 }
 
-// ... or, with the mobilities and mu on the tape, in one launch each
+// ... or, with mu on the tape, in one launch each
 // (chd::adj_march3d, chd::march3d_record)
 static bool adj_march(const ch_sys *s) {
     return adj_split(s) && chd::march3d_ok(s->p) && s->d.model == CH_SIMPLE_WERTHEIM &&
            chd::march3d_reverse_better(s->p, s->d.precision);
 }
 
-// Tape slots: psi_t, and with the three-launch reverse step also mu_t and the
-// mobilities of psi_t behind it (the recompute's two-launch step computes
-// them on its way to psi_{t+1}, so the reverse step reads them back).
-static size_t tape_slot(const ch_sys *s) { return s->bins * s->elt * (adj_split(s) ? 3 : 1); }
+// Tape slots: psi_t, and with these reverse steps also mu_t (two launches: and the
+// mobilities of psi_t) behind it; the recorded step computes them on its way to
+// psi_{t+1}, and the reverse step reads them back.
+static size_t tape_slot(const ch_sys *s) { return s->bins * s->elt * (adj_split(s) ? (adj_march(s) ? 2 : 3) : 1); }
 
 // one recorded state: psi_{t+1} = step(psi_t) from the slot at `in` into `out`
 static hipError_t tape_step1(ch_sys *s, const void *in, void *out, hipStream_t st) {
@@ -1740,7 +1740,7 @@ static hipError_t tape_step1(ch_sys *s, const void *in, void *out, hipStream_t s
     if(adj_split(s)) {
         const size_t fb = s->bins * s->elt;
         if(adj_march(s))
-            return chd::march3d_record(s->p, d.precision, d.mobility, in, out, (char *)in + fb, (char *)in + 2 * fb, st);
+            return chd::march3d_record(s->p, d.precision, d.mobility, in, out, (char *)in + fb, st);
         return chd::stencil_split3d(s->p, d.precision, d.integrator, d.model, d.mobility, in, out, (char *)in + fb,
                                     (char *)in + 2 * fb, st);
     }
@@ -1785,7 +1785,7 @@ extern "C" ch_status ch_sys_record(ch_sys *s, int64_t nsteps, int32_t ckpt_every
     // and the state after the last window; the pseudospectral full tape also
     // keeps the final state
     const int64_t tape_fields = s->rec_full_tape ? nsteps + (ps ? 1 : 0) : 2 * s->rec_window + (ps ? 0 : 1);
-    if(adj_split(s) && !adj_march(s))
+    if(adj_split(s))
         for(void *&b : s->adj_split)
             if(!b && hipMalloc(&b, fb) != hipSuccess) {
                 b = nullptr;
@@ -1891,7 +1891,11 @@ static ch_status adjoint_core(ch_sys *s, double *grads) {
             }
             else {
                 HIPCHK(c, tape_steps(s, tape, 0, len - 1, s->aux));
-                if(adj_split(s)) {
+                if(adj_march(s)) {
+                    // mu of the window's last state
+                    HIPCHK(c, tape_step1(s, field_at(tape, len - 1, tape_slot(s)), s->adj_split[0], s->aux));
+                }
+                else if(adj_split(s)) {
                     // mu and the mobilities of the window's last state
                     char *last = field_at(tape, len - 1, tape_slot(s));
                     HIPCHK(c, chd::split3d_mu(s->p, s->d.precision, s->d.integrator, s->d.model, s->d.mobility, last,
@@ -1913,7 +1917,7 @@ static ch_status adjoint_core(ch_sys *s, double *grads) {
             for(int64_t t = len - 1; t >= 0; t--) {
                 char *slot = field_at(tape, t, tape_slot(s));
                 if(adj_march(s)) {
-                    const void *const rec[3] = {slot, slot + fb, slot + 2 * fb};
+                    const void *const rec[2] = {slot, slot + fb};
                     HIPCHK(c, chd::adj_march3d(s->p, s->d.precision, s->d.mobility, s->lam[li], s->lam[li ^ 1], rec,
                                                s->gacc, ms));
                     li ^= 1;

@@ -46,10 +46,10 @@ hipError_t stencil_march3d(const Params &p, int precision, int integrator, int m
                            void *out, hipStream_t s);
 bool march3d_reverse_better(const Params &p, int precision);
 // SimpleWertheim euler_mobility where march3d_ok and adjoint_split3d_ok
-hipError_t march3d_record(const Params &p, int precision, int mob, const void *in, void *out, void *mu, void *mobs,
+hipError_t march3d_record(const Params &p, int precision, int mob, const void *in, void *out, void *mu,
                           hipStream_t s);
 hipError_t adj_march3d(const Params &p, int precision, int mob, const void *lam_in, void *lam_out,
-                       const void *const slot[3], double *gacc, hipStream_t s);
+                       const void *const slot[2], double *gacc, hipStream_t s);
 inline int stencil_max_k(int dims, int N) { return (dims == 2 && N >= 64) ? 8 : 1; }
 // one euler_mobility step with conserved noise (noise.hip), in -> out; the
 // step index is *step_base + step_off.  noise_step_advance adds n to *step_base.

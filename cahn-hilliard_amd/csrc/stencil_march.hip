@@ -46,11 +46,10 @@ __device__ __forceinline__ void perimeter(int s, int o, int &lx, int &ly) {
     }
 }
 
-// REC: mu and (density-dependent mobility) the mobilities of the old state go to
-// mu_out and mob_out, for the reverse step
+// REC: mu of the old state goes to mu_out, for the reverse step
 template <typename T, int MODEL, int MOB, bool EM, int TX, int TY, int ZC, int NT, bool REC>
 __global__ __launch_bounds__(NT) void k_march3d(const T *__restrict__ in, T *__restrict__ out, Params p, int tiles_x,
-                                                int tiles_y, T *__restrict__ mu_out, T *__restrict__ mob_out) {
+                                                int tiles_y, T *__restrict__ mu_out) {
     constexpr int RX = TX + 4, RY = TY + 4, R = RX * RY;
     constexpr int NI = TX * TY, NU = (TX + 2) * (TY + 2);  // updated cells, mu cells of a plane
     static_assert(R <= NT && NI % 64 == 0, "one thread per cell of the plane, whole waves of updated cells");
@@ -108,10 +107,8 @@ __global__ __launch_bounds__(NT) void k_march3d(const T *__restrict__ in, T *__r
             }
         }
         if(j < ZC + 2) P[(j + 1) & 1][t] = psi[j + 1];
-        if(REC && j >= 2 && j < ZC + 2 && upd) {
+        if(REC && j >= 2 && j < ZC + 2 && upd)
             *reinterpret_cast<T *>(reinterpret_cast<char *>(mu_out + plane(j)) + at) = mu;
-            if constexpr(VARM) *reinterpret_cast<T *>(reinterpret_cast<char *>(mob_out + plane(j)) + at) = mob;
-        }
         if(j >= 3 && upd) {
             const T Um[3] = {Uj[t - 1], Uj[t - RX], um}, Uq[3] = {Uj[t + 1], Uj[t + RX], mu};
             T r;
@@ -137,21 +134,21 @@ __global__ __launch_bounds__(NT) void k_march3d(const T *__restrict__ in, T *__r
 }
 
 template <typename T, int MODEL, int MOB, bool EM, int TX, int TY, int ZC, int NT, bool REC>
-static hipError_t march_cfg(const Params &p, const T *in, T *out, T *mu, T *mobs, hipStream_t s) {
+static hipError_t march_cfg(const Params &p, const T *in, T *out, T *mu, hipStream_t s) {
     const int tiles_x = p.N / TX, tiles_y = p.N / TY;
     hipLaunchKernelGGL((k_march3d<T, MODEL, MOB, EM, TX, TY, ZC, NT, REC>), dim3(tiles_x * tiles_y * (p.N / ZC)),
-                       dim3(NT), 0, s, in, out, p, tiles_x, tiles_y, mu, mobs);
+                       dim3(NT), 0, s, in, out, p, tiles_x, tiles_y, mu);
     return hipGetLastError();
 }
 
 template <typename T, int MODEL, int MOB, bool EM, bool REC = false>
-static hipError_t march_t(const Params &p, const void *in, void *out, hipStream_t s, void *mu = nullptr,
-                          void *mobs = nullptr) {
+static hipError_t march_t(const Params &p, const void *in, void *out, hipStream_t s,
+                          void *mu = nullptr) {
     const T *a = (const T *)in;
-    T *b = (T *)out, *u = (T *)mu, *m = (T *)mobs;
-    if(p.N >= 128) return march_cfg<T, MODEL, MOB, EM, 32, 16, 8, 768, REC>(p, a, b, u, m, s);
-    if(p.N >= 64) return march_cfg<T, MODEL, MOB, EM, 32, 8, 4, 448, REC>(p, a, b, u, m, s);
-    return march_cfg<T, MODEL, MOB, EM, 32, 8, 2, 448, REC>(p, a, b, u, m, s);
+    T *b = (T *)out, *u = (T *)mu;
+    if(p.N >= 128) return march_cfg<T, MODEL, MOB, EM, 32, 16, 8, 768, REC>(p, a, b, u, s);
+    if(p.N >= 64) return march_cfg<T, MODEL, MOB, EM, 32, 8, 4, 448, REC>(p, a, b, u, s);
+    return march_cfg<T, MODEL, MOB, EM, 32, 8, 2, 448, REC>(p, a, b, u, s);
 }
 
 template <typename T, int MODEL>
@@ -170,25 +167,25 @@ static hipError_t march_model(const Params &p, int integrator, int mob, const vo
 // ---- the euler_mobility reverse step in one launch, marching the same way:
 // nu = D(Mob, lambda) of plane j on the region and its first ring, eta and the
 // Laplacian of psi of plane j, and lambda_n of plane j - 1 share a phase.  lambda,
-// psi, mu and the mobilities are read once and lambda_n written, where the
-// two-launch form (k_adj_split_nu, k_adj_split_upd in stencil_split.hip) also
-// writes nu and reads lambda and nu again; the cells' arithmetic is the same
-// (adjoint_math.h), so lambda has the same bits, and only the order of the FP64
-// gradient sums differs.
+// psi and mu are read once and lambda_n written, the mobilities evaluated again from
+// psi (the same function: the same bits; 3 to 14 operations against a third field on
+// the tape, N = 128 linear M 54 -> 47 us), where the two-launch form (k_adj_split_nu,
+// k_adj_split_upd in stencil_split.hip) also reads the mobilities, writes nu and
+// reads lambda and nu again; the cells' arithmetic is the same (adjoint_math.h), so
+// lambda has the same bits, and only the order of the FP64 gradient sums differs.
 // us per reverse step on MI355X, two launches -> this (linear M; constant M):
-//   FP64  N = 32 16.0 -> 7.0; 10.7 -> 6.8   N = 64 13.2 -> 10.3; 11.7 -> 9.2   N = 128 55.8 -> 54.1; 47.3 -> 38.6
-//   FP32  N = 32  9.1 -> 6.5;  8.5 -> 6.4   N = 64  9.0 -> 8.9;  8.1 -> 8.2    N = 128 26.7 -> 35.1; 24.7 -> 30.4
-// and the recorded step, FP64 linear M, 8.0 -> 5.4, 8.9 -> 7.2, 29.9 -> 24.5.  In FP32 the
+//   FP64  N = 32 16.0 -> 6.9; 8.9 -> 6.1   N = 64 12.8 -> 9.8; 11.6 -> 8.8   N = 128 52.6 -> 47.3; 46.2 -> 39.2
+//   FP32  N = 32  7.7 -> 5.8; 6.9 -> 5.7   N = 64  8.6 -> 8.7;  8.2 -> 7.9   N = 128 25.7 -> 27.1; 21.7 -> 24.1
+// and the recorded step, FP64 linear M, 8.0 -> 5.1, 8.9 -> 7.2, 29.4 -> 24.3.  In FP32 the
 // two launches' bytes halve and the FP64 derivatives do not, so from N = 128 on
 // they stay (march3d_reverse_better).  Bound by the FP64 cells and, with one
 // block per CU, by the wait for its first loads.  Blocks as the forward's: at N =
-// 64 FP64 linear M 32 x 8 x 4 10.4, x 2 11.0, x 8 13.0, 32 x 16 x 4 12.8, 32 x 4 x 4 11.8;
-// at N = 128 32 x 16 x 8 54.1, x 4 54.1, 32 x 8 x 8 57.6, x 4 56.4.
+// 64 FP64 linear M 32 x 8 x 4 9.7, x 2 10.6, x 8 12.5, 32 x 16 x 4 12.2, 64 x 4 x 8 12.8;
+// at N = 128 (linear; constant) 32 x 16 x 8 46; 39, x 4 47; 44, 32 x 8 x 8 51; 38, x 16 40; 43.
 template <typename T, int MODEL, int MOB, int TX, int TY, int ZC, int NT>
 __global__ __launch_bounds__(NT) void k_adj_march3d(const T *__restrict__ lam, const T *__restrict__ psi,
-                                                    const T *__restrict__ mu, const T *__restrict__ mob,
-                                                    T *__restrict__ lam_out, Params p, int tiles_x, int tiles_y,
-                                                    double *__restrict__ gacc) {
+                                                    const T *__restrict__ mu, T *__restrict__ lam_out, Params p,
+                                                    int tiles_x, int tiles_y, double *__restrict__ gacc) {
     constexpr int RX = TX + 4, RY = TY + 4, R = RX * RY;
     constexpr int NI = TX * TY, NU = (TX + 2) * (TY + 2);  // updated cells, nu cells of a plane
     static_assert(R <= NT && NI % 64 == 0, "one thread per cell of the plane, whole waves of updated cells");
@@ -218,37 +215,39 @@ __global__ __launch_bounds__(NT) void k_adj_march3d(const T *__restrict__ lam, c
         return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(f + plane(j)) + at);
     };
     const T inv_dx2 = (T)p.inv_dx2, Mc = (T)p.M;
-    T l[ZC + 4], m[ZC + 4], u[ZC + 4], c[ZC + 4];
+    T l[ZC + 4], u[ZC + 4], c[ZC + 4];
 #pragma unroll
     for(int j = 0; j < ZC + 4; j++) {
         l[j] = load(lam, j);
-        if constexpr(VARM) m[j] = load(mob, j);
-        else m[j] = Mc;
+        if(VARM || (j > 0 && j < ZC + 3)) c[j] = load(psi, j);
     }
     if(wave_nu) {
 #pragma unroll
-        for(int j = 1; j < ZC + 3; j++) {
-            u[j] = load(mu, j);
-            c[j] = load(psi, j);
-        }
+        for(int j = 1; j < ZC + 3; j++) u[j] = load(mu, j);
     }
     T num = 0, nuc = 0, etac = 0, lpsc = 0;
     double ge = 0, gk = 0, gm = 0, gd = 0;
     L[1][t] = l[1];
-    if constexpr(VARM) M[1][t] = m[1];
+    T mm = Mc, mc = Mc;  // mobilities of planes j - 1 and j
+    if constexpr(VARM) {
+        mm = mobility<T, MOB>(p, c[0]);
+        mc = mobility<T, MOB>(p, c[1]);
+        M[1][t] = mc;
+    }
     lds_barrier();
 #pragma unroll
     for(int j = 1; j < ZC + 3; j++) {
         const T *Lj = L[j & 1], *Mj = M[VARM ? j & 1 : 0], *Uj = U[j & 1], *Sj = S[j & 1], *Vp = V[(j - 1) & 1];
-        T nu = 0, eta = 0, lps = 0;
+        T nu = 0, eta = 0, lps = 0, mq = Mc;
+        if constexpr(VARM) mq = mobility<T, MOB>(p, c[j + 1]);
         if(wave_nu) {
             const T lm[3] = {Lj[tc - 1], Lj[tc - RX], l[j - 1]}, lq[3] = {Lj[tc + 1], Lj[tc + RX], l[j + 1]};
             T Mm[3] = {Mc, Mc, Mc}, Mq[3] = {Mc, Mc, Mc};
             if constexpr(VARM) {
-                Mm[0] = Mj[tc - 1], Mm[1] = Mj[tc - RX], Mm[2] = m[j - 1];
-                Mq[0] = Mj[tc + 1], Mq[1] = Mj[tc + RX], Mq[2] = m[j + 1];
+                Mm[0] = Mj[tc - 1], Mm[1] = Mj[tc - RX], Mm[2] = mm;
+                Mq[0] = Mj[tc + 1], Mq[1] = Mj[tc + RX], Mq[2] = mq;
             }
-            nu = adj_nu<T, 3>(l[j], m[j], lm, lq, Mm, Mq, inv_dx2);
+            nu = adj_nu<T, 3>(l[j], mc, lm, lq, Mm, Mq, inv_dx2);
             V[j & 1][t] = nu;
             if(upd && j >= 2 && j < ZC + 2) {
                 const T um[3] = {Uj[t - 1], Uj[t - RX], u[j - 1]}, uq[3] = {Uj[t + 1], Uj[t + RX], u[j + 1]};
@@ -263,7 +262,7 @@ __global__ __launch_bounds__(NT) void k_adj_march3d(const T *__restrict__ lam, c
         }
         if(j < ZC + 2) {
             L[(j + 1) & 1][t] = l[j + 1];
-            if constexpr(VARM) M[(j + 1) & 1][t] = m[j + 1];
+            if constexpr(VARM) M[(j + 1) & 1][t] = mq;
         }
         if(j >= 3 && upd) {
             const T nm[3] = {Vp[t - 1], Vp[t - RX], num}, nq[3] = {Vp[t + 1], Vp[t + RX], nu};
@@ -279,6 +278,8 @@ __global__ __launch_bounds__(NT) void k_adj_march3d(const T *__restrict__ lam, c
                 gd += (double)nuc * dfprime_ddelta<MODEL>(p, ps) + (double)etac * md.ddelta;
         }
         if(j < ZC + 2) lds_barrier();
+        mm = mc;
+        mc = mq;
         num = nuc;
         nuc = nu;
         etac = eta;
@@ -289,30 +290,28 @@ __global__ __launch_bounds__(NT) void k_adj_march3d(const T *__restrict__ lam, c
 }
 
 template <typename T, int MODEL, int MOB, int TX, int TY, int ZC, int NT>
-static hipError_t adj_march_cfg(const Params &p, const void *const f[4], void *lam_out, double *gacc, hipStream_t s) {
+static hipError_t adj_march_cfg(const Params &p, const void *const f[3], void *lam_out, double *gacc, hipStream_t s) {
     const int tiles_x = p.N / TX, tiles_y = p.N / TY;
     hipLaunchKernelGGL((k_adj_march3d<T, MODEL, MOB, TX, TY, ZC, NT>), dim3(tiles_x * tiles_y * (p.N / ZC)), dim3(NT), 0,
-                       s, (const T *)f[0], (const T *)f[1], (const T *)f[2], (const T *)f[3], (T *)lam_out, p, tiles_x,
-                       tiles_y, gacc);
+                       s, (const T *)f[0], (const T *)f[1], (const T *)f[2], (T *)lam_out, p, tiles_x, tiles_y, gacc);
     return hipGetLastError();
 }
 
 template <typename T, int MOB>
-static hipError_t adj_march_t(const Params &p, const void *const f[4], void *lam_out, double *gacc, hipStream_t s) {
+static hipError_t adj_march_t(const Params &p, const void *const f[3], void *lam_out, double *gacc, hipStream_t s) {
     constexpr int MODEL = CH_SIMPLE_WERTHEIM;
     if(p.N >= 128) return adj_march_cfg<T, MODEL, MOB, 32, 16, 8, 768>(p, f, lam_out, gacc, s);
     if(p.N >= 64) return adj_march_cfg<T, MODEL, MOB, 32, 8, 4, 448>(p, f, lam_out, gacc, s);
     return adj_march_cfg<T, MODEL, MOB, 32, 8, 2, 448>(p, f, lam_out, gacc, s);
 }
 
-// one recorded step of a system that adj_march3d sweeps back: psi_{t+1}, mu_t and
-// the mobilities of psi_t
-hipError_t march3d_record(const Params &p, int precision, int mob, const void *in, void *out, void *mu, void *mobs,
+// one recorded step of a system that adj_march3d sweeps back: psi_{t+1} and mu_t
+hipError_t march3d_record(const Params &p, int precision, int mob, const void *in, void *out, void *mu,
                           hipStream_t s) {
     auto go = [&](auto mt) {
         constexpr int MOB = decltype(mt)::value;
-        return precision == CH_FP64 ? march_t<double, CH_SIMPLE_WERTHEIM, MOB, true, true>(p, in, out, s, mu, mobs)
-                                    : march_t<float, CH_SIMPLE_WERTHEIM, MOB, true, true>(p, in, out, s, mu, mobs);
+        return precision == CH_FP64 ? march_t<double, CH_SIMPLE_WERTHEIM, MOB, true, true>(p, in, out, s, mu)
+                                    : march_t<float, CH_SIMPLE_WERTHEIM, MOB, true, true>(p, in, out, s, mu);
     };
     switch(mob) {
     case CH_MOB_CONSTANT: return go(std::integral_constant<int, CH_MOB_CONSTANT>{});
@@ -322,10 +321,10 @@ hipError_t march3d_record(const Params &p, int precision, int mob, const void *i
     return hipErrorInvalidValue;
 }
 
-// the reverse step: `slot` as march3d_record leaves it, {psi, mu, mobilities}
+// the reverse step: `slot` as march3d_record leaves it, {psi, mu}
 hipError_t adj_march3d(const Params &p, int precision, int mob, const void *lam_in, void *lam_out,
-                       const void *const slot[3], double *gacc, hipStream_t s) {
-    const void *const f[4] = {lam_in, slot[0], slot[1], slot[2]};
+                       const void *const slot[2], double *gacc, hipStream_t s) {
+    const void *const f[3] = {lam_in, slot[0], slot[1]};
     auto go = [&](auto mt) {
         constexpr int MOB = decltype(mt)::value;
         return precision == CH_FP64 ? adj_march_t<double, MOB>(p, f, lam_out, gacc, s)
