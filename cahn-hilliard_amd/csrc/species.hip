@@ -18,12 +18,14 @@
 //     f', mu_s = f'_s - 2 k_s lap rho_s) then k_sp_update (rho_s += dt M lap mu_s,
 //     or the flux form with M_s per species), in place: 2 launches per step
 //     (EulerCPU.cpp:18-36, EulerMobilityCPU.cpp:31-83 over species);
-//   pseudospectral: k_sp_fprime, then per species r2c, k_sp_ps_update (k_s in
+//   pseudospectral: k_sp_fprime, then per species r2c, k_sp_ps_update (2D: both and
+//                   the column transforms in k_sp_ps_col; k_s in
 //     the denominator, PseudospectralCPU.cpp:112-136) and c2r.
 #include <algorithm>
 #include <cmath>
 
 #include "ch_internal.h"
+#include "line_fft.h"
 
 namespace chd {
 
@@ -451,25 +453,80 @@ __global__ __launch_bounds__(256) void k_sp_mob(const T *__restrict__ rho, const
 #undef SP_CELLS
 
 // the pseudospectral update of one species (PseudospectralCPU.cpp:118-133)
+// one spectral entry of the semi-implicit update; k_s in the denominator
+template <typename T>
+__device__ __forceinline__ void sp_ps_entry(const Params &p, double ks, int ix, int iy, int iz, C2<T> f, C2<T> &r, C2<T> &out) {
+#pragma clang fp contract(off)
+    double k2, deal;
+    mode_q2(p, ix, iy, iz, k2, deal);
+    if(p.use_dealias) f = C2<T>{f.x * (T)deal, f.y * (T)deal};
+    const double k4 = k2 * k2;
+    const T den = (T)(1.0 + p.dt * p.M * (p.S * k2 + 2.0 * ks * k4));
+    const T a = (T)(p.dt * p.M * k2), S = (T)p.S, ib = (T)p.inv_bins;
+    const T re = (r.x - a * (f.x - S * r.x)) / den;
+    const T im = (r.y - a * (f.y - S * r.y)) / den;
+    r = C2<T>{re, im};
+    out = C2<T>{re * ib, im * ib};
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void k_sp_ps_update(C2<T> *__restrict__ rh, C2<T> *__restrict__ fh,
                                                       C2<T> *__restrict__ copy, Params p, int64_t hat, double ks) {
-#pragma clang fp contract(off)
     for(int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < hat; q += (int64_t)gridDim.x * 256) {
         int ix, iy, iz;
         mode_index(p, q, ix, iy, iz);
-        double k2, deal;
-        mode_q2(p, ix, iy, iz, k2, deal);
-        C2<T> f = fh[q];
-        if(p.use_dealias) f = C2<T>{f.x * (T)deal, f.y * (T)deal};
-        const double k4 = k2 * k2;
-        const T den = (T)(1.0 + p.dt * p.M * (p.S * k2 + 2.0 * ks * k4));
-        const T a = (T)(p.dt * p.M * k2), S = (T)p.S, ib = (T)p.inv_bins;
-        const C2<T> r = rh[q];
-        const T re = (r.x - a * (f.x - S * r.x)) / den;
-        const T im = (r.y - a * (f.y - S * r.y)) / den;
-        rh[q] = C2<T>{re, im};
-        copy[q] = C2<T>{re * ib, im * ib};
+        C2<T> r = rh[q], o;
+        sp_ps_entry<T>(p, ks, ix, iy, iz, fh[q], r, o);
+        rh[q] = r;
+        copy[q] = o;
+    }
+}
+
+// 2D up to N = 2048: the column transforms around the update in one pass (the line
+// engines of line_fft.h), three launches per species for five, each a start and a
+// round trip to what the other XCDs wrote.  Saleh, FP64 on MI355X, us per step, with
+// the row passes' smaller blocks (line_fft.h): N = 64 71.0 -> 42.7, 256 82.3 -> 49.2,
+// 512 93.8 -> 67.3, 1024 162 -> 108; Generic N = 256 237 -> 66.6 (its sweeps, too).
+template <typename T, class ENG>
+__global__ __launch_bounds__(ENG::NT) void k_sp_ps_col(const C2<T> *__restrict__ in, C2<T> *__restrict__ out,
+                                                       C2<T> *__restrict__ rho_hat, const C2<T> *__restrict__ table, Params p,
+                                                       int lines, double ks) {
+    constexpr int E = ENG::E, Nh = ENG::n / 2 + 1;
+    __shared__ typename ENG::Smem sm;
+    const int l0 = xcd_tile(blockIdx.x, gridDim.x) * ENG::NL;
+    if(l0 >= lines) return;  // grid padded to a multiple of 8 blocks
+    ENG eng(sm);
+    eng.begin(table);
+    const bool on = ENG::NL == 1 || l0 + eng.line() < lines;
+    const int l = on ? l0 + eng.line() : l0;
+    C2<T> v[E], rh[E];
+#pragma unroll
+    for(int i = 0; i < E; i++) v[i] = in[(size_t)eng.in(i) * Nh + l];
+#pragma unroll
+    for(int i = 0; i < E; i++) rh[i] = rho_hat[(size_t)eng.freq(i) * Nh + l];
+    eng.finish(table);
+    eng.forward(v);
+#pragma unroll
+    for(int i = 0; i < E; i++) sp_ps_entry<T>(p, ks, l, eng.freq(i), 0, v[i], rh[i], v[i]);
+    eng.inverse(v);
+#pragma unroll
+    for(int i = 0; i < E; i++)
+        if(on) {
+            rho_hat[(size_t)eng.freq(i) * Nh + l] = rh[i];
+            out[(size_t)eng.in(i) * Nh + l] = v[i];
+        }
+}
+
+template <typename T, int LOG2N = 2>
+static hipError_t sp_ps_col(const SpectralArgs &a, const C2<T> *in, C2<T> *out, C2<T> *rh, double ks, hipStream_t s) {
+    if constexpr(LOG2N > 11) return hipErrorInvalidValue;
+    else {
+        if(a.p.log2N != LOG2N) return sp_ps_col<T, LOG2N + 1>(a, in, out, rh, ks, s);
+        using Eng = Engine<T, LOG2N, 2>;
+        constexpr int lines = (1 << LOG2N) / 2 + 1;
+        hipLaunchKernelGGL((k_sp_ps_col<T, Eng>), dim3(col_blocks(lines, Eng::NL)), dim3(Eng::NT), 0, s, in, out, rh,
+                           (const C2<T> *)a.twiddles, a.p, lines, ks);
+        return hipGetLastError();
     }
 }
 
@@ -668,6 +725,13 @@ hipError_t sp_step_spectral(const SpArgs &a, const SpectralArgs &sa, hipStream_t
             SpectralArgs b = sa;
             b.rho = (T *)a.rho + sp * a.bins;
             C2<T> *rh = (C2<T> *)a.rho_hat + sp * a.hat;
+            if(a.p.dims == 2 && a.p.N <= 2048) {
+                e = spec_x_forward(b, (const T *)a.mu + sp * a.bins, a.spec[0], false, s);
+                if(e == hipSuccess)
+                    e = sp_ps_col<T>(b, (const C2<T> *)a.spec[0], (C2<T> *)a.spec[1], rh, a.m_host->k[sp], s);
+                if(e == hipSuccess) e = spec_x_inverse(b, a.spec[1], (T *)a.rho + sp * a.bins, s);
+                continue;
+            }
             e = spec_r2c(b, (const T *)a.mu + sp * a.bins, a.spec[0], false, s);
             if(e != hipSuccess) break;
             hipLaunchKernelGGL((k_sp_ps_update<T>), dim3(grid_for(a.hat)), dim3(256), 0, s, rh, (C2<T> *)a.spec[0],
