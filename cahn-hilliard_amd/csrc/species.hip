@@ -18,9 +18,9 @@
 //     f', mu_s = f'_s - 2 k_s lap rho_s) then k_sp_update (rho_s += dt M lap mu_s,
 //     or the flux form with M_s per species), in place: 2 launches per step
 //     (EulerCPU.cpp:18-36, EulerMobilityCPU.cpp:31-83 over species);
-//   pseudospectral: k_sp_fprime, then per species r2c, k_sp_ps_update (2D: both and
-//                   the column transforms in k_sp_ps_col; k_s in
-//     the denominator, PseudospectralCPU.cpp:112-136) and c2r.
+//   pseudospectral: k_sp_fprime, then per species r2c, the update (k_s in the
+//     denominator, PseudospectralCPU.cpp:112-136) and c2r; in 2D the columns'
+//     transforms and the update are one pass (k_sp_ps_col), else k_sp_ps_update.
 #include <algorithm>
 #include <cmath>
 
