@@ -67,7 +67,9 @@ struct SpectralArgs {
     void *rho_hat;        // half spectrum state (T2)
     const void *twiddles; // W_N^m, m = 0..N-1 (T2)
     // rho_hat may be stored line-major (entry j of column line l at l N + j; 2D N =
-    // 256 to 2048): set for the pseudospectral integrator, whose chain alone reads it
+    // 256 to 2048): set for the pseudospectral integrator, whose chain alone reads
+    // that field.  rho_hat is then a buffer of its own: the pass that stores it
+    // reads work, so the two must not be the same (fft2_forward clears this)
     bool rh_lines = false;
 };
 // init = true: rho_hat = r2c(rho); otherwise one time step

@@ -1162,6 +1162,10 @@ static hipError_t fft2_inverse_p(const SpectralArgs &a, void *out, hipStream_t s
 hipError_t fft2_forward(const SpectralArgs &a, hipStream_t s) {
     SpectralArgs b = a;
     b.rho_hat = a.work;  // the forward r2c of ps_run's set-up, written into work
+    // the columns are transformed in place, and the shells and the inverse read the
+    // half spectrum's own layout: line-major stores would land on lines that
+    // other blocks have not read yet
+    b.rh_lines = false;
     return ps_run(b, s, true);
 }
 
