@@ -248,6 +248,17 @@ static chd::Params make_params(const ch_desc *d) {
     p.M = d->M;
     p.rho_min = d->rho_min;
     p.rho_ref = d->rho_ref;
+    // the linear rule's divisor and its reciprocal; extreme ones are brought to where
+    // the reciprocal is normal, by one power of two with the numerator's factor
+    auto linear = [&](auto one, auto far, auto up) {
+        using T = decltype(one);
+        const T b = (T)d->rho_ref, ab = std::fabs(b), sc = ab < one / far ? up : (ab > far ? one / up : one);
+        p.lin_M = (T)d->M * sc;
+        p.lin_ref = b * sc;
+        p.lin_inv = one / (b * sc);
+    };
+    if(d->precision == CH_FP64) linear(1.0, 0x1p900, 0x1p200);
+    else linear(1.0f, 0x1p100f, 0x1p60f);
     p.k = d->k;
     p.two_k = 2.0 * d->k;
     p.dx = d->dx;

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void k_mob_max(const T *__restrict__ rho, T *_
     __shared__ double red[256];
     double m = 0.0;
     for(int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < bins; i += (int64_t)gridDim.x * 256) {
-        const T v = mobility<T, MOB>(p, rho[i]);
+        const T v = mobility_divided<T, MOB>(p, rho[i]);
         mob[i] = v;
         m = (double)v > m ? (double)v : m;
     }

@@ -283,7 +283,7 @@ __global__ void k_fprime(const T *__restrict__ in, T *__restrict__ out, Params p
 template <typename T, int MOB>
 __global__ void k_mobility(const T *__restrict__ in, T *__restrict__ out, Params p, int64_t n) {
     for(int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        out[i] = mobility<T, MOB>(p, in[i]);
+        out[i] = mobility_divided<T, MOB>(p, in[i]);
 }
 
 static int grid_for(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 8192)); }
