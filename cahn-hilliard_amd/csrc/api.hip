@@ -410,10 +410,12 @@ extern "C" ch_status ch_sys_create(ch_ctx *ctx, const ch_desc *desc, ch_sys **ou
     if(const char *tb = std::getenv("CH_TB_STEPS")) want = std::atoi(tb);
     s->tb = 1;
     while(s->tb * 2 <= max_k && s->tb * 2 <= want) s->tb *= 2;
-    // grids that one block holds, and 1D: many steps per launch (CH_TB_STEPS pins
-    // the depth of the other kernels instead)
-    if(!is_spectral(desc->integrator) && !noisy && !std::getenv("CH_TB_STEPS"))
-        s->multi = chd::stencil_multi_steps(desc->dims, N);
+    // grids that one block holds, and 1D: many steps per launch.  Pins of the other
+    // kernels' depth (CH_TB_STEPS), region shape (CH_WAVE_CFG) or tile (CH_TILE3D) run
+    // those kernels instead
+    const bool pinned = std::getenv("CH_TB_STEPS") || (desc->dims == 2 && N >= 64 && std::getenv("CH_WAVE_CFG")) ||
+                        (desc->dims == 3 && std::getenv("CH_TILE3D"));
+    if(!is_spectral(desc->integrator) && !noisy && !pinned) s->multi = chd::stencil_multi_steps(desc->dims, N);
     if(const char *r = std::getenv("CH_WAVE_CFG")) s->p.wave_cfg = std::max(0, std::min(chd::kWaveCfgs - 1, std::atoi(r)));
     // N >= 1024: 128 x 80 regions for the launches shorter than 8 steps (measured at N = 1024
     // with 8-step launches and a 4-step tail: 0.2635 ms per 100 steps against
