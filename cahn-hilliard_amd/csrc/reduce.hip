@@ -280,10 +280,18 @@ __global__ void k_fprime(const T *__restrict__ in, T *__restrict__ out, Params p
         out[i] = fprime<T, MODEL>(p, in[i]);
 }
 
+// M rho X^valence for valence < 1: no system's descriptor has one, but ch_set_mobility
+// takes any
+__device__ __forceinline__ double unbonded_mobility(const Params &p, double r) {
+#pragma clang fp contract(off)
+    const double D = pow_uniform(wertheim_X(p, r), -p.valence);
+    return r * (p.M * (p.valence == 0 ? 1.0 : 1.0 / D));
+}
+
 template <typename T, int MOB>
 __global__ void k_mobility(const T *__restrict__ in, T *__restrict__ out, Params p, int64_t n) {
     for(int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        out[i] = mobility_divided<T, MOB>(p, in[i]);
+        out[i] = MOB == CH_MOB_FREE_ENERGY && p.valence < 1 ? (T)unbonded_mobility(p, (double)in[i]) : mobility_divided<T, MOB>(p, in[i]);
 }
 
 static int grid_for(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 8192)); }
