@@ -285,9 +285,12 @@ static chd::Params make_params(const ch_desc *d) {
     if(split) p.tile3d = 3;
     if(d->dims == 3 && chd::march3d_better(p, d->precision, d->integrator, d->model, d->mobility)) p.tile3d = split ? 5 : 4;
     p.adj_tile3d = 1;
-    // noise step tiles: 64 x 32 in 2D from N = 1024, else 64 x 16 (twice the
-    // blocks) and 8 x 8 x 8 in 3D, all with 512 threads (figures in noise.hip)
-    p.noise_tile = d->dims == 2 && d->N >= 1024 ? 2 : 1;
+    // noise step tiles, all with 512 threads (figures in noise.hip): 64 x 32 in 2D from
+    // N = 1024, else 64 x 16 (twice the blocks); in 3D 8 x 8 x 8, but 16 x 8 x 8 where a
+    // density-dependent mobility is one more field in LDS: from N = 64, in FP32 from 128
+    const bool var_mob = d->mobility != CH_MOB_CONSTANT;
+    const bool wide = d->dims == 2 ? d->N >= 1024 : var_mob && d->N >= (d->precision == CH_FP64 ? 64 : 128);
+    p.noise_tile = wide ? 2 : 1;
     p.S = d->S;
     double bins = std::pow((double)d->N, d->dims);
     p.vbin_over_bins = d->dx * d->dx * d->dx / bins;

@@ -21,7 +21,7 @@ struct Params {
     int adj_cfg;           // region shape of the 2D wave adjoint (0, 3, 4, 5 or 9)
     int tile3d;            // 3D forward step: LDS tile 0: 16x8x8 / 256 threads, 1: the same / 512, 2: 16x16x4 / 512; 3: two launches (stencil_split.hip); 4, 5: one launch marching along z (stencil_march.hip; 5: the reverse step in two launches)
     int adj_tile3d;        // 3D tile of the euler_mobility adjoint (0: 16x4x4 / 256, 1 (default): 16x8x4 / 512, 2: 16x8x8 / 512)
-    int noise_tile;        // tile of the noise step (0: 2D 64x16, 3D 8x8x8 / 256 threads; 1 (default): the same / 512; 2 (default for 2D N >= 1024): 2D 64x32, 3D 16x8x8 / 512)
+    int noise_tile;        // tile of the noise step (0: 2D 64x16, 3D 8x8x8 / 256 threads; 1: the same / 512; 2: 2D 64x32, 3D 16x8x8 / 512; chosen in make_params)
     double eps;            // Landau epsilon
     double B2, reg, log_reg, tvd;   // SimpleWertheim: tvd = 2 valence delta
     double M, rho_min, rho_ref;     // mobility

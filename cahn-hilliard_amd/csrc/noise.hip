@@ -245,7 +245,13 @@ hipError_t launch_noise_cfg(const Params &p, const void *in, void *out, const in
 //   2D N = 256  64 x 16 / 512 threads 5.3, 64 x 32 / 512 7.1     N = 512  5.7, 7.4
 //      N = 1024 12.9, 11.1    N = 2048 42.9, 40.4
 //   3D N = 32   8 x 8 x 8 / 512 5.9, 16 x 8 x 8 / 512 8.7        N = 64   8.7, 8.9
-//      N = 128  51.0, 60.2 (FP32 32.7, 32.2)
+//      N = 128  51.0, 60.2 (FP32 32.0, 32.1)
+// and with a density-dependent mobility, whose LDS field leaves 8 x 8 x 8 one block fewer
+// per CU, 3D SimpleWertheim linear mobility (Landau regularised):
+//      N = 32   8 x 8 x 8 / 512 7.3 (6.8), 16 x 8 x 8 / 512 11.0 (10.1)
+//      N = 64   12.6 (11.6), 11.1 (10.0)    FP32 8.3 (7.4), 9.1 (7.9)
+//      N = 128  89.5 (83.2), 78.1 (69.3)    FP32 45.2 (39.1), 43.9 (38.0)
+//      N = 256  720 (667), 623 (556)        FP32 336 (297), 339 (298)
 // Rows of a tile per wave instead of indexed loops: fewer instructions, but no
 // faster (2D N = 1024 13.2): the rounds of rows leave waves idle.
 template <typename T, int DIMS, int MODEL, int MOB>
