@@ -83,27 +83,34 @@ __device__ __forceinline__ void sincos_2pi(double u, double &sn, double &cs) {
     cs = __builtin_fma(ck, cr, -(sk * sr));
 }
 
-// the same in FP32: r = f pi / 4 with f exact, series through r^7 and r^8 (first
-// omitted terms below 3e-9), where sincosf of the rounded product 2 pi u reduces
-// a general argument
+// the same in FP32 by quadrants: 4 u = q + f, f exact in [-1/2, 1/2], the series of
+// sin and cos of f pi / 2 through f^9 and f^10 (first omitted terms below 2e-9), pi / 2
+// split into its FP32 value and the rest; no rotation by the octant's angle and
+// fewer selects than octants take.  Every 97th u2 against FP64: at most 6.1e-8 off
+// (octants 1.07e-7, sincosf of the rounded product 2 pi u 4.1e-7).  3D Landau with
+// regularised mobility, 16 x 8 x 8 tiles, us per step with octants -> this (with signs by
+// selects in place of xor): N = 128 39.0 -> 35.5 (37.5), N = 256 296 -> 276 (292).
 __device__ __forceinline__ void sincos_2pi(float u, float &sn, float &cs) {
 #pragma clang fp contract(off)
-    const float v = 8.0f * u;
-    const int k = (int)v;
-    const float r = ((v - (float)k) - 0.5f) * 0.78539816339744830962f;
-    const float t = r * r;
-    float s = fma_t(fma_t(-1.0f / 5040.0f, t, 1.0f / 120.0f), t, -1.0f / 6.0f);
-    const float sr = fma_t(r * t, s, r);
-    float c = fma_t(fma_t(fma_t(1.0f / 40320.0f, t, -1.0f / 720.0f), t, 1.0f / 24.0f), t, -0.5f);
-    const float cr = fma_t(t, c, 1.0f);
-    constexpr float S1 = 0.38268343236508977173f, C1 = 0.92387953251128675613f;  // sin, cos of pi/8
-    const int o = k & 7;  // u = 1 after rounding: octant 8
-    const bool swap = o == 1 || o == 2 || o == 5 || o == 6;
-    float sk = swap ? C1 : S1, ck = swap ? S1 : C1;
-    if(o >= 4) sk = -sk;
-    if(o >= 2 && o <= 5) ck = -ck;
-    sn = fma_t(sk, cr, ck * sr);
-    cs = fma_t(ck, cr, -(sk * sr));
+    constexpr double h = 1.57079632679489661923, h2 = h * h, h4 = h2 * h2, h8 = h4 * h4;
+    const float v = 4.0f * u, q = __builtin_rintf(v), f = v - q;
+    const int k = (int)q;  // 0 .. 4
+    const float t = f * f;
+    float s = (float)(h8 * h / 362880);
+    s = fma_t(s, t, (float)(-h4 * h2 * h / 5040));
+    s = fma_t(s, t, (float)(h4 * h / 120));
+    s = fma_t(s, t, (float)(-h2 * h / 6));
+    s = fma_t(s, t, (float)(h - (double)(float)h));
+    s = fma_t(f, (float)h, f * s);
+    float c = (float)(-h8 * h2 / 3628800);
+    c = fma_t(c, t, (float)(h8 / 40320));
+    c = fma_t(c, t, (float)(-h4 * h2 / 720));
+    c = fma_t(c, t, (float)(h4 / 24));
+    c = fma_t(c, t, (float)(-h2 / 2));
+    c = fma_t(t, c, 1.0f);
+    const uint32_t a = __builtin_bit_cast(uint32_t, k & 1 ? c : s), b = __builtin_bit_cast(uint32_t, k & 1 ? s : c);
+    sn = __builtin_bit_cast(float, a ^ ((uint32_t)(k & 2) << 30));  // signs
+    cs = __builtin_bit_cast(float, b ^ ((uint32_t)((k + 1) & 2) << 30));
 }
 
 // standard normals DIMS of cell `cell` at step `step`, in T
