@@ -129,7 +129,7 @@ struct PsmArgs {
 };
 // nsteps splitting steps, asynchronous (capturable)
 hipError_t psm_steps_simple(const PsmArgs &B, int64_t nsteps, hipStream_t s);
-// the same in 2D and 3D as fused line passes (psm_pass.hip)
+// the same in 2D (FP64: N <= 1024) and 3D as fused line passes (psm_pass.hip)
 hipError_t psm_chain(const PsmArgs &B, int64_t nsteps, hipStream_t s);
 // the mobility of rho into B.mob, its nparts (<= kPsmParts) partial maxima into `parts`
 hipError_t psm_mobility(const PsmArgs &B, double *parts, int &nparts, hipStream_t s);

@@ -12,8 +12,8 @@
 //             / (1 + dt M0 (S q^2 + 2k q^4));   rho = c2r(rho_hat) / N^d
 // Everything stays on the device (M0 included), so a chain of steps is
 // captured into a graph like the other integrators.  In 2D and 3D the chain
-// runs as fused line passes (psm_pass.hip); 1D, and CH_PSM_FUSE=0, as the
-// element-wise kernels below around whole transforms.
+// runs as fused line passes (psm_pass.hip); 1D, FP64 2D from N = 2048, and
+// CH_PSM_FUSE=0, as the element-wise kernels below around whole transforms.
 //
 // Full scheme (_evolve_full, :303-404): A x = b with
 //   A x = x - dt div(M grad((S - 2k lap) x)),  b = rho + dt div(M grad(f' - S rho)),
@@ -357,11 +357,17 @@ struct Ops {
         return e;
     }
 
+    // The fused passes where they are the faster form.  A 2D FP64 grid from N = 2048
+    // leaves the caches, and there whole contiguous rows weigh more than launches and
+    // passes: us per step, fused passes -> whole transforms, Landau regularised, 4 and 32
+    // steps per call, N = 2048 391, 372 -> 374, 372, N = 4096 2305, 2257 -> 1994, 1996
+    // (SimpleWertheim linear 417, 400 -> 390, 385 and 2408, 2372 -> 2059, 2056); FP32
+    // 250 -> 305, 1108 -> 1263, 3D N = 256 FP64 1697 -> 2207
+    bool chain_better() const { return p().dims == 3 || (p().dims == 2 && (sizeof(T) == 4 || p().N < 2048)); }
+
     hipError_t steps_simple(int64_t nsteps) {
         hipError_t e = hipSuccess;
-        if(B.fuse && p().dims >= 2) {
-            return nsteps < 1 ? e : psm_chain(B, nsteps, s);
-        }
+        if(B.fuse && chain_better()) return nsteps < 1 ? e : psm_chain(B, nsteps, s);
         for(int64_t i = 0; i < nsteps && e == hipSuccess; i++) e = step_simple();
         return e;
     }

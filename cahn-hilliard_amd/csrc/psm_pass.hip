@@ -505,7 +505,7 @@ hipError_t chain_n(const PsmArgs &B, int64_t nsteps, hipStream_t s) {
     case 9: return Chain<T, 9, DIMS>(B, s).run(nsteps);
     case 10: return Chain<T, 10, DIMS>(B, s).run(nsteps);
     }
-    if constexpr(DIMS == 2) {
+    if constexpr(DIMS == 2 && sizeof(T) == 4) {  // FP64: psm.hip's whole transforms are faster there
         if(B.a.p.log2N == 11) return Chain<T, 11, 2>(B, s).run(nsteps);
         if(B.a.p.log2N == 12) return Chain<T, 12, 2>(B, s).run(nsteps);
     }
