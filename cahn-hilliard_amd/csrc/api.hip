@@ -1332,6 +1332,7 @@ static constexpr int kBatchDepths = 4;
 struct ch_batch {
     ch_ctx *ctx = nullptr;
     int n = 0, precision = CH_FP64, model = CH_LANDAU, graph_steps = 0;
+    int64_t max_bins = 0;  // cells of the largest replica
     int tb = 4, shape = 0;  // steps per launch and region split (autotuned)
     bool tuned = false;     // false: tune on the first evolve
     size_t elt = 8;
@@ -1489,7 +1490,6 @@ extern "C" ch_status ch_batch_create_ex(ch_ctx *ctx, int32_t n, const ch_desc *d
         if(esh) b->shape = std::max(0, std::min(chd::kBatchShapes - 1, std::atoi(esh)));
     }
     std::vector<int2> items[chd::kBatchFamilies][kBatchDepths];
-    int64_t maxbins = 0;
     for(int r = 0; r < n; r++) {
         chd::BatchRep rep{};
         rep.p = make_params(&descs[r]);
@@ -1501,7 +1501,7 @@ extern "C" ch_status ch_batch_create_ex(ch_ctx *ctx, int32_t n, const ch_desc *d
                 for(int code : chd::batch_items(chd::batch_family_shape(fam), N, 1 << i))
                     items[fam][i].push_back(int2{r, code});
         b->total += (int64_t)N * N;
-        maxbins = std::max<int64_t>(maxbins, (int64_t)N * N);
+        b->max_bins = std::max<int64_t>(b->max_bins, (int64_t)N * N);
         b->host_reps.push_back(rep);
     }
     const char *g = std::getenv("CH_GRAPH_STEPS");
@@ -1510,7 +1510,7 @@ extern "C" ch_status ch_batch_create_ex(ch_ctx *ctx, int32_t n, const ch_desc *d
     if(!b->tuned && tune_lookup(tune_key(b), b->shape, b->tb)) b->tuned = true;
     bool ok = hipMalloc(&b->buf[0], b->total * b->elt) == hipSuccess && hipMalloc(&b->buf[1], b->total * b->elt) == hipSuccess &&
               hipMalloc((void **)&b->reps, n * sizeof(chd::BatchRep)) == hipSuccess &&
-              hipMalloc(&b->stage, maxbins * 8) == hipSuccess && hipMalloc((void **)&b->result, 2 * (size_t)n * (1 + chd::kBatchObsParts) * sizeof(double)) == hipSuccess;
+              hipMalloc(&b->stage, b->max_bins * 8) == hipSuccess && hipMalloc((void **)&b->result, 2 * (size_t)n * (1 + chd::kBatchObsParts) * sizeof(double)) == hipSuccess;
     if(ok && (compensation == CH_COMP_STORED || compensation == CH_COMP_LOW8)) {
         const size_t bytes = b->total * b->comp_elt();
         ok = hipMalloc(&b->comp[0], bytes) == hipSuccess && hipMalloc(&b->comp[1], bytes) == hipSuccess &&
@@ -1701,7 +1701,7 @@ extern "C" ch_status ch_batch_observables(ch_batch *b, double *mass, double *fre
     if(!b) return CH_EINVAL;
     ch_ctx *c = b->ctx;
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, chd::batch_observables(b->precision, b->model, b->buf[b->cur], b->reps, b->n, b->result, c->stream));
+    HIPCHK(c, chd::batch_observables(b->precision, b->model, b->buf[b->cur], b->reps, b->n, b->max_bins, b->result, c->stream));
     std::vector<double> h(2 * (size_t)b->n);
     HIPCHK(c, hipMemcpyAsync(h.data(), b->result, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));

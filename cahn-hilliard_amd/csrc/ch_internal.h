@@ -230,10 +230,11 @@ std::vector<int> batch_items(int shape, int N, int K);  // tx | ty << 16 per ite
 hipError_t batch_launch(int precision, int model, int upd, int shape, int K, const void *a, void *b,
                         const BatchRep *reps, const int2 *items, int nitems, const void *ca, void *cb, hipStream_t s);
 // per-replica FP64 observables: result[2 r] = sum rho, result[2 r + 1] = sum f-density
-// result: 2 n (1 + kBatchObsParts) values, the sums of each replica and then scratch
+// result: 2 n (1 + kBatchObsParts) values, the sums of each replica and then scratch;
+// max_bins: the cells of the largest replica
 constexpr int kBatchObsParts = 32;
-hipError_t batch_observables(int precision, int model, const void *buf, const BatchRep *reps, int n, double *result,
-                             hipStream_t s);
+hipError_t batch_observables(int precision, int model, const void *buf, const BatchRep *reps, int n, int64_t max_bins,
+                             double *result, hipStream_t s);
 
 // adjoint (adjoint.hip).  `em`: the euler_mobility integrator (any mobility
 // rule); otherwise euler with constant mobility.  Every adjoint tile owns

@@ -216,11 +216,12 @@ hipError_t finalize_pairs(double *partials, int nparts, double *result, hipStrea
     return hipGetLastError();
 }
 
-// kBatchObsParts blocks per replica of a batch (one where the replicas alone fill
-// the chip), each over a contiguous part of its cells, then one wave per replica
-// for the parts.  One block per replica left the
-// largest one's cells to four waves: a call for 64 replicas of N = 64 to 512 in
-// FP32 took 360 us, now 43; 4 of N = 1024 1340, now 70.
+// kBatchObsParts blocks per replica of a batch, each over a contiguous part of its
+// cells, then one wave per replica for the parts; one block, straight to the result, where
+// the replicas alone fill the chip, or are Landau's of N = 64, whose cells take less
+// than the second launch.  us per call, one block -> parts, FP32: 64 replicas of N = 64
+// to 512 360 -> 43, 4 of N = 1024 784 -> 62, 8 of N = 64 28.6 -> 29.4 (SimpleWertheim 36.3
+// -> 29.4), 1500 of N = 64 37 (40 with a second launch for one part each).
 template <typename T, int MODEL>
 __global__ __launch_bounds__(256) void k_batch_obs(const T *__restrict__ buf, const BatchRep *__restrict__ reps,
                                                    double *__restrict__ parts, int np) {
@@ -257,10 +258,10 @@ __global__ __launch_bounds__(64) void k_batch_obs_final(const double *__restrict
     }
 }
 
-hipError_t batch_observables(int precision, int model, const void *buf, const BatchRep *reps, int n, double *result,
-                             hipStream_t s) {
-    double *parts = result + 2 * (size_t)n;
-    const int np = n < 1024 ? kBatchObsParts : 1;
+hipError_t batch_observables(int precision, int model, const void *buf, const BatchRep *reps, int n, int64_t max_bins,
+                             double *result, hipStream_t s) {
+    const int np = n >= 1024 || (model == CH_LANDAU && max_bins <= 64 * 64) ? 1 : kBatchObsParts;
+    double *parts = np == 1 ? result : result + 2 * (size_t)n;
     auto go = [&](auto t) {
         using T = decltype(t);
         const dim3 grid((unsigned)n * np);
@@ -269,7 +270,7 @@ hipError_t batch_observables(int precision, int model, const void *buf, const Ba
     };
     if(precision == CH_FP64) go(double{});
     else go(float{});
-    hipLaunchKernelGGL(k_batch_obs_final, dim3(n), dim3(64), 0, s, parts, result, np);
+    if(np > 1) hipLaunchKernelGGL(k_batch_obs_final, dim3(n), dim3(64), 0, s, parts, result, np);
     return hipGetLastError();
 }
 
