@@ -278,8 +278,9 @@ static chd::Params make_params(const ch_desc *d) {
     p.adj_cfg = chd::adj_default_cfg(d->N);
     // 3D steps below N = 32: LDS tiles of 16x8x8 with 512 threads, or for
     // SimpleWertheim the two-launch step, which evaluates each cell's FP64 f'
-    // once; from N = 32 one launch marching along z (4; 5 where the reverse step
-    // runs in two launches, as with the two-launch forward)
+    // once; from N = 32 one launch marching along z where it is the faster form
+    // (march3d_better): 4, or 5 where split3d_ok, whose reverse step marches too (two
+    // launches in FP32 from N = 128)
     p.tile3d = 1;
     const bool split = d->dims == 3 && d->model == CH_SIMPLE_WERTHEIM && chd::split3d_ok(p, d->integrator, d->mobility);
     if(split) p.tile3d = 3;

@@ -19,7 +19,7 @@ struct Params {
     int use_dealias;
     int wave_cfg;          // region shape of the 2D wave kernel (0 .. kWaveCfgs - 1)
     int adj_cfg;           // region shape of the 2D wave adjoint (0, 3, 4, 5 or 9)
-    int tile3d;            // 3D forward step: LDS tile 0: 16x8x8 / 256 threads, 1: the same / 512, 2: 16x16x4 / 512; 3: two launches (stencil_split.hip); 4, 5: one launch marching along z (stencil_march.hip; 5: the reverse step in two launches)
+    int tile3d;            // 3D forward step: LDS tile 0: 16x8x8 / 256 threads, 1: the same / 512, 2: 16x16x4 / 512; 3: two launches (stencil_split.hip); 4, 5: one launch marching along z (stencil_march.hip; 5: the reverse step too, in FP32 below N = 128)
     int adj_tile3d;        // 3D tile of the euler_mobility adjoint (0: 16x4x4 / 256, 1 (default): 16x8x4 / 512, 2: 16x8x8 / 512)
     int noise_tile;        // tile of the noise step (0: 2D 64x16, 3D 8x8x8 / 256 threads; 1: the same / 512; 2: 2D 64x32, 3D 16x8x8 / 512; chosen in make_params)
     double eps;            // Landau epsilon
@@ -447,6 +447,11 @@ constexpr int kWaveCfgs = 10;
 //   SimpleWertheim euler     9/8         9/8         9/4         5/4         5/2         5/2
 //                            2.30, 3.07  2.30, 3.07  3.33, 3.58  7.19, 7.98  24.7, 28.8  81.8, 99.4
 //     free-energy mobility   3.45, 4.82  3.45, 4.82  4.83, 5.57  8.98, 10.5  29.3, 38.2  99.8, 130
+// and in FP32, the same rule against the same alternatives:
+//   Landau euler             0.93, 1.05  0.95, 1.06  1.10        1.81        4.58        12.6, 14.0
+//   Landau, regularised      1.30, 1.72  1.35, 1.73  1.83        3.90        10.9, 12.1  30.6, 39.5
+//   SimpleWertheim euler     2.19, 2.91  2.30, 2.94  2.97, 3.13  6.69, 7.81  21.0, 26.1  68.4, 91.1
+//     free-energy mobility   3.21, 4.58  3.30, 4.59  4.18, 4.79  8.31, 9.90  26.4, 34.1  89.9, 124
 struct WaveRule {
     int cfg, steps;
 };
@@ -462,7 +467,7 @@ __host__ __device__ constexpr WaveRule wave_default(int N, bool wertheim, bool v
 // reverse sweep and its forward recompute (shapes 0, 3, 4, 5, 9): 128 x 64 regions
 // from N = 512; 64 x 40 at N = 128 and 256, where 64 x 64 leaves three CUs in four
 // idle (record of every 16th state + sweep of 64 steps in FP64, N = 256: 386 -> 356 us,
-// every state kept 282 -> 254); 64 x 64, the whole grid, at 64
+// every state kept 282 -> 254; FP32 359 -> 355, 253 -> 241); 64 x 64, the whole grid, at 64
 __host__ __device__ constexpr int adj_default_cfg(int N) {
     return N >= 512 ? 5 : (N >= 128 ? 9 : 4);
 }
