@@ -125,7 +125,7 @@ __device__ __forceinline__ void cell_normals(uint64_t seed, uint32_t cell, uint6
         if constexpr(sizeof(T) == 8) {
             const double u1 = ((double)w[2 * h] + 0.5) * 0x1p-32;
             const double u2 = ((double)w[2 * h + 1] + 0.5) * 0x1p-32;
-            const double r = sqrt_normal(-2.0 * log_series_pos(u1));  // 4.6e-10 .. 46
+            const double r = sqrt_normal(-2.0 * log_series_pos(u1));  // 2.3e-10 .. 46
             double sn, cs;
             sincos_2pi(u2, sn, cs);
             eta[2 * h] = r * cs;
