@@ -23,16 +23,16 @@
 //                       FP32   4.0 / 4.8  5.3 / 5.1 14.9 / 13.5   103 / 90
 //            free-energy M FP64 4.9 / 7.3 6.9 / 7.3 22.3 / 31.9   128 / 215
 // and in FP32, march, LDS tile, two launches (measured side by side):
-//   Wertheim, linear M         4.4, 6.6, 6.0   5.8, 6.4, 6.2   15.9, 21.7, 15.6   99.9, 142, 96.7
-//            regularised M     4.5, 6.6, 6.0   6.0, 6.4, 6.2   16.7, 22.2, 15.7   107, 150, 98.4
+//   Wertheim, linear M         4.4, 6.6, 6.0   5.8, 6.4, 6.2   15.7, 21.7, 15.6   93.8, 142, 98.7
+//            regularised M     4.5, 6.6, 6.0   6.0, 6.4, 6.2   16.3, 22.2, 15.6   98.5, 150, 101
 //            free-energy M     4.7, 6.8, 9.9   6.1, 6.7, 9.4   16.6, 23.2, 24.2   101, 160, 169
 //            constant M        4.3, 6.2, 5.1   5.5, 6.1, 5.4   15.1, 20.2, 13.4   91.5, 136, 80.3
-// FP32 SimpleWertheim moves half the bytes for the same FP64 f', so there the
-// launch that evaluates f' once per cell stays ahead from N = 64 with constant mobility
-// and from N = 128 with a linear or regularised one; the free-energy rule, as dear as f', is
-// evaluated with it (march3d_better).  Chunks of 8 planes from N = 128 (16: 8.9 us for
-// Landau FP32, fewer blocks than the CUs hold), 32 x 8 x 4 at N = 64 and 32 x 8
-// x 2 at N = 32, where smaller blocks fill more CUs.
+// FP32 SimpleWertheim with constant mobility moves half the bytes for the same
+// FP64 f', so there the launch that evaluates f' once per cell stays ahead from
+// N = 64 (march3d_better); with the other rules the march is ahead or level but
+// for the regularised one at N = 128 (six runs in both orders).  Chunks of 8 planes
+// from N = 128 (16: 8.9 us for Landau FP32, fewer blocks than the CUs hold), 32 x 8 x 4
+// at N = 64 and 32 x 8 x 2 at N = 32, where smaller blocks fill more CUs.
 #include "adjoint_math.h"
 #include "ch_internal.h"
 
@@ -347,8 +347,8 @@ hipError_t adj_march3d(const Params &p, int precision, int mob, const void *lam_
 
 bool march3d_better(const Params &p, int precision, int integrator, int model, int mob) {
     if(p.N < 32) return false;
-    if(precision == CH_FP64 || model != CH_SIMPLE_WERTHEIM || mob == CH_MOB_FREE_ENERGY) return true;
-    return p.N < (integrator == CH_EULER || mob == CH_MOB_CONSTANT ? 64 : 128);
+    const bool constant = integrator == CH_EULER || mob == CH_MOB_CONSTANT;
+    return !(precision == CH_FP32 && model == CH_SIMPLE_WERTHEIM && constant && p.N >= 64);
 }
 
 bool march3d_reverse_better(const Params &p, int precision) { return precision == CH_FP64 || p.N < 128; }
